@@ -139,6 +139,16 @@ int iris_hip_gemm_fill(const iris_gemm_problem_t *problem, float *d_workspace, s
 int iris_hip_gemm_fill_n(const iris_gemm_problem_t *problems, int n_problems, float *d_workspace,
                          size_t workspace_bytes);
 
+/* No counterpart in the reference. The launch on tiles of 64 or 128 rows by
+ * 128 columns whose loads run in waves of their own, several K steps ahead:
+ * what iris_hip_gemm_fill and _fill_n take for products of at most 128 rows
+ * (a short prompt, a caption) and, unsplit, for one whose 128 x 128 tiles
+ * fill most of one round. splits and the workspace as iris_hip_gemm_splitk
+ * (every problem split alike); results equal it and iris_hip_gemm bit for
+ * bit. No second K segment. */
+int iris_hip_gemm_ring(const iris_gemm_problem_t *problems, int n_problems, int rows, int splits, float *d_workspace,
+                       size_t workspace_bytes);
+
 /* No counterpart in the reference. iris_hip_gemm_splitk without a
  * workspace, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc): the

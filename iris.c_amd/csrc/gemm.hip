@@ -766,6 +766,261 @@ __global__ __launch_bounds__(NT) void gemm_bf16_kernel(const GemmParams P) {
     }
 }
 
+/* Products on few rows: block tiles of 32 FM x 32 FN over a ring of NS LDS
+ * stages, 8 waves: waves 0..3 compute (2x2, wave tile 16 FM x 16 FN), waves
+ * 4..7 only load, one of each on a SIMD. The K step of a small tile is bound
+ * by issue, not by its products: a wave that issues an LDS-DMA load waits for
+ * the address unit (16 clocks per 1 KiB load), so where the computing waves
+ * also load, a step takes the sum of its load issue, products and fragment
+ * reads; with waves of their own the loads cost the products nothing, and
+ * NS - 1 steps are in flight (72 to 120 KiB per CU) against the latency of
+ * weights that come from HBM.
+ *
+ * One barrier per K step. A computing wave runs step t's first 32-wide half
+ * on fragments read during step t-1 while it reads the second half's, meets
+ * the barrier when its reads of tile t are done, then reads tile t+1's first
+ * half while the second half's products run. A loading wave meets step t's
+ * barrier when its loads of tile t+1 are done (loads of a wave complete in
+ * order: the count of the younger ones is enough), then issues tile t+NS into
+ * the stage of tile t. Past the last tile it repeats tile nk-1 into stages
+ * nothing reads again. Every output element gets the additions of the kernel
+ * above in its order. */
+template <int FM_, int FN_, int NS>
+__global__ __launch_bounds__(512) void gemm_ring_kernel(const GemmParams P) {
+    constexpr int BMR = 32 * FM_, BNR = 32 * FN_, TM = 16 * FM_, TN = 16 * FN_;
+    constexpr int A_DMA = BMR / DMA_ROWS / 4, W_DMA = BNR / DMA_ROWS / 4, LD = A_DMA + W_DMA;
+    constexpr int A_ELEMS = BMR * BK, ST_ELEMS = (BMR + BNR) * BK;
+    static_assert(NS >= 3 && (NS - 1) * LD < 64, "ring depth");
+    extern __shared__ __attribute__((aligned(16))) uint16_t ring[];
+    const int L = (blockIdx.x & 7) * P.per_xcd + (blockIdx.x >> 3);
+    if (L >= P.total) return;
+    int pi = 0;
+#pragma unroll
+    for (int i = 1; i < MAXP; i++)
+        if (i < P.nprob && L >= P.tile_start[i]) pi = i;
+    iris_gemm_problem_t pr = P.p[pi];
+    int t = L - P.tile_start[pi];
+    if (P.chunks[pi] > 1) {
+        const int per = P.tiles_m[pi] * P.tiles_n[pi];
+        const int chunk = __builtin_amdgcn_readfirstlane(t / per), k0 = chunk * P.kchunk[pi];
+        t -= chunk * per;
+        pr.A += k0;
+        pr.W += k0;
+        pr.K = min(P.kchunk[pi], pr.K - k0);
+        pr.out = P.ws[pi] + chunk * P.ws_stride[pi];
+        pr.ldo = pr.N;
+        pr.vec = nullptr;
+        pr.epi = IRIS_EPI_F32;
+    }
+    const int tmc = P.tiles_m[pi], tnc = P.tiles_n[pi];
+    /* scalar registers for what the buffer resources are made of */
+    const int first_m = __builtin_amdgcn_readfirstlane(t / (GROUP_M * tnc)) * GROUP_M;
+    const int gsz = min(tmc - first_m, GROUP_M), tg = t - first_m * tnc;
+    const int tn = __builtin_amdgcn_readfirstlane(tg / gsz);
+    const int m0 = (first_m + tg - tn * gsz) * BMR, n0 = tn * BNR;
+
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = (wave >> 1) & 1, wn = wave & 1;
+    const int nk = pr.K / BK;
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (wave >= 4) {
+        const int lw = wave & 3;
+        const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(pr.A + (size_t)m0 * pr.lda), (short)0, min(BMR, pr.M - m0) * pr.lda * 2, 0x00020000);
+        const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(pr.W + (size_t)n0 * pr.ldw), (short)0, min(BNR, pr.N - n0) * pr.ldw * 2, 0x00020000);
+        /* load j of an operand covers tile rows 8j .. 8j+7; loading wave w
+         * issues loads j = DMA w .. + DMA - 1; lane l fetches row 8j + l/8,
+         * chunk (l%8) ^ ((row >> 1) & 7) */
+        const int drow = lane >> 3, dch = lane & 7;
+        int a_voff[2], w_voff[2];
+#pragma unroll
+        for (int par = 0; par < 2; par++) {
+            const int ca = dch ^ ((4 * ((par + (A_DMA & 1) * lw) & 1) + (drow >> 1)) & 7);
+            const int cw = dch ^ ((4 * ((par + (W_DMA & 1) * lw) & 1) + (drow >> 1)) & 7);
+            a_voff[par] = ((lw * A_DMA * DMA_ROWS + drow) * pr.lda + ca * 8) * 2;
+            w_voff[par] = ((lw * W_DMA * DMA_ROWS + drow) * pr.ldw + cw * 8) * 2;
+        }
+        const int a_step = DMA_ROWS * pr.lda * 2, w_step = DMA_ROWS * pr.ldw * 2;
+        auto dma = [&](int stage, int kt) {
+            const int soff = kt * BK * 2;
+            uint16_t *const st = ring + stage * ST_ELEMS;
+#pragma unroll
+            for (int i = 0; i < W_DMA; i++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(st + A_ELEMS + (lw * W_DMA + i) * 512),
+                                                         16, w_voff[i & 1] + i * w_step, soff, 0, 0);
+#pragma unroll
+            for (int i = 0; i < A_DMA; i++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_void *)(st + (lw * A_DMA + i) * 512), 16,
+                                                         a_voff[i & 1] + i * a_step, soff, 0, 0);
+        };
+        for (int i = 0; i < NS; i++) dma(i, min(i, nk - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 1) * LD, 15));
+        barrier();
+        for (int kt = 0, st = 0; kt < nk; kt++) {
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * LD, 15));
+            barrier();
+            dma(st, min(kt + NS, nk - 1));
+            st = st == NS - 1 ? 0 : st + 1;
+        }
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));   /* no DMA outstanding at exit */
+        return;
+    }
+
+    f32x4 acc[FM_][FN_];
+#pragma unroll
+    for (int i = 0; i < FM_; i++)
+#pragma unroll
+        for (int j = 0; j < FN_; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[i][j][r] = 0.0f;
+    bf16x8 a0[FM_], w0[FN_], a1[FM_], w1[FN_];
+    /* rows 16 apart keep their swizzle: one base per half */
+    const int ab0 = swz(wm * TM + lr, lg), wb0 = A_ELEMS + swz(wn * TN + lr, lg);
+    const int ab1 = swz(wm * TM + lr, 4 + lg), wb1 = A_ELEMS + swz(wn * TN + lr, 4 + lg);
+    auto frags = [&](int st, int ab, int wb, bf16x8 (&a)[FM_], bf16x8 (&w)[FN_]) {
+#pragma unroll
+        for (int mi = 0; mi < FM_; mi++) a[mi] = *(const bf16x8 *)(ring + st + ab + mi * 16 * BK);
+#pragma unroll
+        for (int ni = 0; ni < FN_; ni++) w[ni] = *(const bf16x8 *)(ring + st + wb + ni * 16 * BK);
+    };
+    auto mfmas = [&](const bf16x8 (&a)[FM_], const bf16x8 (&w)[FN_]) {
+#pragma unroll
+        for (int mi = 0; mi < FM_; mi++)
+#pragma unroll
+            for (int ni = 0; ni < FN_; ni++)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[ni], a[mi], acc[mi][ni], 0, 0, 0);
+    };
+    /* a fragment read between products, whose operands are in registers */
+    auto interleave = [&]() {
+#pragma unroll
+        for (int i = 0; i < FM_ + FN_; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+    };
+    barrier();   /* tile 0 */
+    frags(0, ab0, wb0, a0, w0);
+    for (int kt = 0, st = 0; kt < nk; kt++) {
+        frags(st, ab1, wb1, a1, w1);
+        mfmas(a0, w0);
+        interleave();
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
+        barrier();   /* tile kt + 1 is there, tile kt is read */
+        st = st == (NS - 1) * ST_ELEMS ? 0 : st + ST_ELEMS;
+        frags(st, ab0, wb0, a0, w0);
+        mfmas(a1, w1);
+        interleave();
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    /* lane l holds row lr of each 16x16 tile at the 4 columns lg*4 .. lg*4+3 */
+    const int M = pr.M, N = pr.N, ldo = pr.ldo;
+    const float *vec = pr.vec;
+    const bool aligned = (ldo & 3) == 0 && ((uintptr_t)pr.out & 15) == 0 && ((uintptr_t)vec & 15) == 0;
+    if (pr.epi == IRIS_EPI_SWIGLU) {
+        /* 64 columns of the wave are 32 gate rows, then the matching 32 up rows */
+#pragma unroll
+        for (int g = 0; g < FN_ / 4; g++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int col = ((n0 + wn * TN + g * 64) >> 1) + h * 16 + lg * 4;
+                if (col >= (N >> 1)) continue;   /* N % 64 == 0: all four columns or none */
+#pragma unroll
+                for (int mi = 0; mi < FM_; mi++) {
+                    const int row = m0 + wm * TM + mi * 16 + lr;
+                    if (row >= M) continue;
+                    const f32x4 gt = acc[mi][4 * g + h], up = acc[mi][4 * g + 2 + h];
+                    uint16_t y[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) y[r] = f2bf_hw(silu_fast(gt[r]) * up[r]);
+                    uint16_t *dst = (uint16_t *)pr.out + (size_t)row * ldo + col;
+                    if (aligned) {
+                        *(uint2 *)dst = make_uint2((uint32_t)y[0] | ((uint32_t)y[1] << 16),
+                                                   (uint32_t)y[2] | ((uint32_t)y[3] << 16));
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; r++) dst[r] = y[r];
+                    }
+                }
+            }
+        return;
+    }
+#pragma unroll
+    for (int ni = 0; ni < FN_; ni++) {
+        const int col = n0 + wn * TN + ni * 16 + lg * 4;
+        const bool cols4 = aligned && col + 3 < N;
+        const float vdef = pr.epi == IRIS_EPI_GATED_ADD ? 1.0f : 0.0f;
+        float v[4];
+        if (cols4 && vec) {
+            const float4 q = *(const float4 *)(vec + col);
+            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = vec && col + r < N ? vec[col + r] : vdef;
+        }
+#pragma unroll
+        for (int mi = 0; mi < FM_; mi++) {
+            const int row = m0 + wm * TM + mi * 16 + lr;
+            if (row >= M) continue;
+            const f32x4 x = acc[mi][ni];
+            const size_t o = (size_t)row * ldo + col;
+            if (cols4 && pr.epi != IRIS_EPI_F32_T) {
+                if (pr.epi == IRIS_EPI_BF16) {
+                    *(uint2 *)((uint16_t *)pr.out + o) =
+                        make_uint2((uint32_t)f2bf_hw(x[0] + v[0]) | ((uint32_t)f2bf_hw(x[1] + v[1]) << 16),
+                                   (uint32_t)f2bf_hw(x[2] + v[2]) | ((uint32_t)f2bf_hw(x[3] + v[3]) << 16));
+                } else {
+                    float4 *dst = (float4 *)((float *)pr.out + o);
+                    float4 y = make_float4(x[0] + v[0], x[1] + v[1], x[2] + v[2], x[3] + v[3]);
+                    if (pr.epi == IRIS_EPI_GATED_ADD) {
+                        y = *dst;
+                        y.x += v[0] * x[0]; y.y += v[1] * x[1]; y.z += v[2] * x[2]; y.w += v[3] * x[3];
+                    } else if (pr.epi == IRIS_EPI_ADD) {
+                        const float4 q = *dst;
+                        y.x = q.x + y.x; y.y = q.y + y.y; y.z = q.z + y.z; y.w = q.w + y.w;
+                    }
+                    *dst = y;
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    if (col + r >= N) continue;
+                    float *const f = (float *)pr.out + (pr.epi == IRIS_EPI_F32_T ? (size_t)(col + r) * ldo + row : o + r);
+                    const float y = x[r] + v[r];
+                    if (pr.epi == IRIS_EPI_BF16) ((uint16_t *)pr.out)[o + r] = f2bf_hw(y);
+                    else if (pr.epi == IRIS_EPI_GATED_ADD) *f += v[r] * x[r];
+                    else if (pr.epi == IRIS_EPI_ADD) *f += y;
+                    else *f = y;
+                }
+            }
+        }
+    }
+}
+
+/* the tile shapes of gemm_ring_kernel: 6 stages of 24 KiB, 4 of 32 KiB */
+enum { RING_NONE, RING_64, RING_128 };
+constexpr int RING_BM[] = {0, 64, 128}, RING_BN = 128;
+
+template <int FM_, int FN_, int NS> int launch_ring(const dim3 &grid, const GemmParams &P) {
+    constexpr size_t smem = (size_t)NS * 32 * (FM_ + FN_) * BK * 2;
+    static std::once_flag once;
+    static hipError_t attr = hipSuccess;
+    std::call_once(once, [] {
+        attr = hipFuncSetAttribute((const void *)gemm_ring_kernel<FM_, FN_, NS>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    });
+    if (iris_check(attr, "gemm_ring smem attribute")) return -1;
+    IRIS_LAUNCH((gemm_ring_kernel<FM_, FN_, NS>), grid, dim3(512), smem, iris_stream(), P);
+    return 0;
+}
+
 /* Split-K partials of up to MAXP problems, reduced in one launch: each
  * output element is the sum of its problem's partials in chunk order
  * (deterministic), then that problem's epilogue. A thread takes VW = vw[i]
@@ -939,8 +1194,9 @@ namespace {
  * round); bnt > 0 forces the tile width. bmt = 128: 128 x 256 tiles (no
  * second K segment). */
 int launch_gemm(const iris_gemm_problem_t *probs, int n, const int *want, float *ws, size_t ws_bytes,
-                int phase1 = 0, int force_bnt = 0, int bmt = BM) {
+                int phase1 = 0, int force_bnt = 0, int bmt = BM, int ring = RING_NONE) {
     if (!probs || n < 1 || n > MAXP) return iris_set_error("gemm: %d problems (1..%d)", n, MAXP);
+    if (ring) bmt = RING_BM[ring];
     GemmParams P;
     memset(&P, 0, sizeof(P));
     P.nprob = n;
@@ -952,7 +1208,7 @@ int launch_gemm(const iris_gemm_problem_t *probs, int n, const int *want, float 
         P.chunks[i] = 1;
         if (p.M <= 0 || p.N <= 0) continue;
         if (check_problem(p)) return -1;
-        if (bmt != BM && p.K2) return iris_set_error("gemm: 128-row tiles take no second K segment");
+        if (bmt != BM && p.K2) return iris_set_error("gemm: tiles of %d rows take no second K segment", bmt);
         P.tiles_m[i] = (p.M + bmt - 1) / bmt;
         if (want && want[i] > 1) {
             const int nk = p.K / BK;
@@ -983,7 +1239,9 @@ int launch_gemm(const iris_gemm_problem_t *probs, int n, const int *want, float 
     if (t256 == 0) return 0;
     int bnt = BN;
     const int cus = iris_cu_count();
-    if (bmt != BM) {
+    if (ring) {
+        bnt = RING_BN;
+    } else if (bmt != BM) {
         bnt = BN;
     } else if (force_bnt == 224 && !seg2 && !swiglu_tiles) {
         bnt = 224;
@@ -1006,7 +1264,9 @@ int launch_gemm(const iris_gemm_problem_t *probs, int n, const int *want, float 
     }
     P.per_xcd = (total - P.phase_tiles + 7) / 8;
     const dim3 grid(P.phase_blocks + 8 * P.per_xcd);
-    if (bmt != BM)
+    if (ring) {
+        if (ring == RING_64 ? launch_ring<2, 4, 6>(grid, P) : launch_ring<4, 4, 4>(grid, P)) return -1;
+    } else if (bmt != BM)
         IRIS_LAUNCH((gemm_bf16_kernel<0, 256, 128>), grid, dim3(NT), 0, iris_stream(), P);
     else if (bnt == 224)
         IRIS_LAUNCH((gemm_bf16_kernel<0, 224>), grid, dim3(NT), 0, iris_stream(), P);
@@ -1173,6 +1433,62 @@ int tail_plan(const iris_gemm_problem_t &p, size_t ws_bytes, iris_gemm_problem_t
 
 }  // namespace
 
+namespace {
+
+/* The faster plan of gemm_ring_kernel for these problems: at most 128 rows
+ * each, in up to one round of blocks, or one problem whose 128 x 128 tiles
+ * fill most of a round unsplit; K of 2048 and more (32 steps: a shorter K
+ * costs a launch either way, and keeps the chunks of the two-stage plan
+ * whatever the number of rows). Elsewhere its tiles load more bytes per
+ * product than the larger ones and lose (measured, cold weights, us against
+ * the two-stage kernel's plans: 512 x 2560 x 9728 45.7 / 45.4, 768 x 18432 x
+ * 3072 122 / 69). The estimate (us): K steps per block times a step of the
+ * tile, plus launch, prologue and epilogue, plus the reduce pass; not less
+ * than the weights' read at the device's copy rate. Measured against it, us,
+ * cold weights (two-stage plan -> this kernel): 37 rows, N x K 6144 x 2560
+ * 20.4 -> 15.8, 2560 x 4096 19.5 -> 14.8, 19456 x 2560 SwiGLU 32.5 -> 26.1,
+ * 2560 x 9728 26.7 -> 20.8; 96 rows, 3840 x 3840 23.3 -> 18.0; 128 rows,
+ * 2560 x 9728 30.1 -> 24.4; 512 x 6144 x 2560 (192 tiles, no reduce pass)
+ * 39.4 -> 31.6. */
+struct RingPlan {
+    int ring, splits;
+    double us;
+};
+
+RingPlan ring_plan(const iris_gemm_problem_t *probs, int n, int cus, size_t ws_bytes) {
+    RingPlan best = {RING_NONE, 1, 1e30};
+    long long tiles[3] = {0, 0, 0};
+    double per = 0, out = 0, wbytes = 0;
+    int min_nk = 1 << 30, max_nk = 0, max_m = 0;
+    for (int i = 0; i < n; i++) {
+        const iris_gemm_problem_t &p = probs[i];
+        if (p.M <= 0 || p.N <= 0) continue;
+        for (int r = RING_64; r <= RING_128; r++)
+            tiles[r] += (long long)((p.M + RING_BM[r] - 1) / RING_BM[r]) * ((p.N + RING_BN - 1) / RING_BN);
+        per += (double)p.M * p.N * 4;
+        out += (double)p.M * p.N * (p.epi == IRIS_EPI_GATED_ADD || p.epi == IRIS_EPI_ADD ? 8 : 4);
+        wbytes += (double)p.N * p.K * 2;
+        min_nk = std::min(min_nk, p.K / BK);
+        max_nk = std::max(max_nk, p.K / BK);
+        max_m = std::max(max_m, p.M);
+    }
+    for (int r = RING_64; r <= RING_128 && min_nk >= 32; r++) {
+        if (tiles[r] > cus) continue;
+        if (max_m > 128 && (n > 1 || r != RING_128 || tiles[r] * 10 < cus * 6LL)) continue;
+        const int most = max_m > 128 ? 1 : (int)std::min<long long>(cus / tiles[r], min_nk / 4);
+        for (int s = 1; s <= std::max(1, most) && (s == 1 || s * per <= (double)ws_bytes); s++) {
+            const double steps = (max_nk + s - 1) / s;
+            double us = r == RING_64 ? steps * 0.40 + 9.0 : steps * 0.56 + 9.5;
+            us = std::max(us, wbytes / 5.1e6 + 6.0);
+            if (s > 1) us += (s * per + out) / 4.5e6 + 3.5;
+            if (us < best.us) best = {r, s, us};
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
 extern "C" int iris_hip_gemm_fill_n(const iris_gemm_problem_t *probs, int n, float *ws, size_t ws_bytes) {
     if (!probs || n < 1 || n > MAXP) return iris_set_error("gemm_fill: %d problems (1..%d)", n, MAXP);
     const int cus = iris_cu_count();
@@ -1217,6 +1533,11 @@ extern "C" int iris_hip_gemm_fill_n(const iris_gemm_problem_t *probs, int n, flo
         const int s256 = fit(cus / tiles);
         const int s128 = tiles128 <= cus ? fit(cus / tiles128) : 0;
         int want[MAXP];
+        const RingPlan r = ring_plan(probs, n, cus, ws_bytes);
+        if (r.ring && r.us < 0.97 * std::min(est(false, s256), s128 > 0 ? est(true, s128) : 1e30)) {
+            for (int i = 0; i < n; i++) want[i] = r.splits;
+            return launch_gemm(probs, n, r.splits > 1 ? want : nullptr, ws, ws_bytes, 0, 0, BM, r.ring);
+        }
         if (s128 > 0 && est(true, s128) < est(false, s256)) {
             for (int i = 0; i < n; i++) want[i] = s128;
             return launch_gemm(probs, n, s128 > 1 ? want : nullptr, ws, ws_bytes, 0, 0, 128);
@@ -1236,6 +1557,14 @@ extern "C" int iris_hip_gemm_fill_n(const iris_gemm_problem_t *probs, int n, flo
         }
     }
     return launch_gemm(probs, n, nullptr, nullptr, 0);
+}
+
+extern "C" int iris_hip_gemm_ring(const iris_gemm_problem_t *probs, int n, int rows, int splits, float *ws,
+                                  size_t ws_bytes) {
+    if (rows != 64 && rows != 128) return iris_set_error("gemm_ring: tiles of %d rows (64 or 128)", rows);
+    int want[MAXP];
+    for (int i = 0; i < MAXP; i++) want[i] = splits;
+    return launch_gemm(probs, n, splits > 1 ? want : nullptr, ws, ws_bytes, 0, 0, BM, rows == 64 ? RING_64 : RING_128);
 }
 
 extern "C" int iris_hip_gemm_fill(const iris_gemm_problem_t *p, float *ws, size_t ws_bytes) {
