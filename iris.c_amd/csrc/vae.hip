@@ -39,10 +39,10 @@ __device__ __forceinline__ void load8(const uint16_t *p, float v[8]) {
 }
 __device__ __forceinline__ uint4 pack8(const float v[8]) {
     uint4 o;
-    o.x = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
-    o.y = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-    o.z = (uint32_t)f2bf(v[4]) | ((uint32_t)f2bf(v[5]) << 16);
-    o.w = (uint32_t)f2bf(v[6]) | ((uint32_t)f2bf(v[7]) << 16);
+    o.x = (uint32_t)f2bf_hw(v[0]) | ((uint32_t)f2bf_hw(v[1]) << 16);
+    o.y = (uint32_t)f2bf_hw(v[2]) | ((uint32_t)f2bf_hw(v[3]) << 16);
+    o.z = (uint32_t)f2bf_hw(v[4]) | ((uint32_t)f2bf_hw(v[5]) << 16);
+    o.w = (uint32_t)f2bf_hw(v[6]) | ((uint32_t)f2bf_hw(v[7]) << 16);
     return o;
 }
 
@@ -134,13 +134,18 @@ __global__ __launch_bounds__(NT) void gn_finalize_kernel(const double *part, int
 }
 
 /* y = act(x * ab[c] + ab[C + c]) in bf16, act = swish or identity; raw (if
- * not NULL) receives x itself in bf16 (the input of a 1x1 skip convolution). */
+ * not NULL) receives x itself in bf16 (the input of a 1x1 skip convolution).
+ * HBM-bound once its arithmetic is short: the channel of a chunk by a mask (a
+ * 64-bit remainder for channel counts that are no power of two), the hardware
+ * reciprocal and bf16 conversion on values rounded to bf16 next. 1024 x 1024 x 128 bf16:
+ * 129 -> 102 us (5.3 TB/s); f32 in 196 us (4.1 TB/s) before and after. */
 template <typename T>
 __global__ __launch_bounds__(NT) void gn_apply_kernel(const T *x, const float *ab, int C, size_t n8, int swish,
                                                       uint16_t *y, uint16_t *raw) {
     const int cpr = C >> 3;
+    const bool pow2 = (cpr & (cpr - 1)) == 0;
     for (size_t i = (size_t)blockIdx.x * NT + threadIdx.x; i < n8; i += (size_t)gridDim.x * NT) {
-        const int c0 = (int)(i % cpr) * 8;
+        const int c0 = (pow2 ? (int)i & (cpr - 1) : (int)(i % cpr)) * 8;
         float v[8];
         load8(x + i * 8, v);
         if (raw) *(uint4 *)(raw + i * 8) = pack8(v);
@@ -151,7 +156,7 @@ __global__ __launch_bounds__(NT) void gn_apply_kernel(const T *x, const float *a
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const float t = v[j] * a[j] + b[j];
-            v[j] = swish ? silu_f(t) : t;
+            v[j] = swish ? silu_fast(t) : t;
         }
         *(uint4 *)(y + i * 8) = pack8(v);
     }
@@ -162,76 +167,95 @@ __global__ __launch_bounds__(NT) void gn_apply_kernel(const T *x, const float *a
  * x / sc + sh (Z-Image: sc = scaling factor, sh = shift); unpatchify 2x2
  * (channel c * 4 + 2 * (oy & 1) + (ox & 1) at (oy / 2, ox / 2) becomes
  * channel c at (oy, ox)); then the 1x1 post_quant_conv when pqw is not NULL;
- * channels z..63 are zero (conv_in's weights are padded to match). */
+ * channels z..63 are zero (conv_in's weights are padded to match). A block
+ * takes 32 pixels, their z values in LDS, and a thread 8 channels of one
+ * pixel: a thread for all 64 of a pixel left most CUs idle. 64 x 64 latent 42 -> 10 us. */
+constexpr int FR_PIX = NT / 8;
 __global__ __launch_bounds__(NT) void vae_front_kernel(const float *lat, int z, int h, int w, const float *sc,
                                                        const float *sh, int divide, const float *pqw,
                                                        const float *pqb, uint16_t *out) {
-    __shared__ float wsh[32 * 32];
+    __shared__ float wsh[32 * 33], vs[FR_PIX][33];   /* rows one word apart in the banks */
     if (pqw)
-        for (int i = threadIdx.x; i < z * z; i += NT) wsh[i] = pqw[i];
-    __syncthreads();
-    const int W2 = 2 * w, npix = 4 * h * w;
-    const int p = blockIdx.x * NT + threadIdx.x;
-    if (p >= npix) return;
-    const int oy = p / W2, ox = p % W2;
-    float v[32], o[64];
-    for (int c = 0; c < z; c++) {
-        const int ic = c * 4 + (oy & 1) * 2 + (ox & 1);
+        for (int i = threadIdx.x; i < z * z; i += NT) wsh[i / z * 33 + i % z] = pqw[i];
+    const int W2 = 2 * w, npix = 4 * h * w, p0 = blockIdx.x * FR_PIX;
+    for (int i = threadIdx.x; i < FR_PIX * z; i += NT) {
+        const int q = i % FR_PIX, c = i / FR_PIX, p = p0 + q;
+        if (p >= npix) continue;
+        const int oy = p / W2, ox = p % W2, ic = c * 4 + (oy & 1) * 2 + (ox & 1);
         const float x = lat[((size_t)ic * h + (oy >> 1)) * w + (ox >> 1)];
-        v[c] = divide ? x / sc[ic] + sh[ic] : x * sc[ic] + sh[ic];
+        vs[q][c] = divide ? x / sc[ic] + sh[ic] : x * sc[ic] + sh[ic];
     }
-    for (int j = 0; j < 64; j++) o[j] = 0.0f;
-    if (pqw) {
-        for (int j = 0; j < z; j++) {
-            float a = pqb ? pqb[j] : 0.0f;
-            for (int c = 0; c < z; c++) a += wsh[j * z + c] * v[c];
-            o[j] = a;
-        }
-    } else {
-        for (int j = 0; j < z; j++) o[j] = v[j];
-    }
-    uint4 *dst = (uint4 *)(out + (size_t)p * 64);
+    __syncthreads();
+    const int q = threadIdx.x >> 3, j0 = (threadIdx.x & 7) * 8;
+    if (p0 + q >= npix) return;
+    float o[8];
 #pragma unroll
-    for (int k = 0; k < 8; k++) dst[k] = pack8(o + 8 * k);
+    for (int j = 0; j < 8; j++) {
+        o[j] = 0.0f;
+        if (j0 + j >= z) continue;
+        if (pqw) {
+            float a = pqb ? pqb[j0 + j] : 0.0f;
+            for (int c = 0; c < z; c++) a += wsh[(j0 + j) * 33 + c] * vs[q][c];
+            o[j] = a;
+        } else {
+            o[j] = vs[q][j0 + j];
+        }
+    }
+    *(uint4 *)(out + (size_t)(p0 + q) * 64 + j0) = pack8(o);
 }
 
 /* Encoder input: image [3][H][W] f32 (NCHW) -> bf16 [H][W][64], channels
  * 3..63 zero (conv_in's weights are padded to match). */
 __global__ __launch_bounds__(NT) void vae_img_in_kernel(const float *img, int npix, uint16_t *out) {
-    const int p = blockIdx.x * NT + threadIdx.x;
+    /* 8 threads a pixel, one 16-byte chunk each: whole lines per store */
+    const int p = blockIdx.x * (NT / 8) + (threadIdx.x >> 3), k = threadIdx.x & 7;
     if (p >= npix) return;
-    float o[64];
+    float o[8];
 #pragma unroll
-    for (int j = 0; j < 64; j++) o[j] = 0.0f;
-    o[0] = img[p];
-    o[1] = img[(size_t)npix + p];
-    o[2] = img[2 * (size_t)npix + p];
-    uint4 *dst = (uint4 *)(out + (size_t)p * 64);
-#pragma unroll
-    for (int k = 0; k < 8; k++) dst[k] = pack8(o + 8 * k);
+    for (int j = 0; j < 8; j++) o[j] = 0.0f;
+    if (k == 0) {
+        o[0] = img[p];
+        o[1] = img[(size_t)npix + p];
+        o[2] = img[2 * (size_t)npix + p];
+    }
+    *(uint4 *)(out + (size_t)p * 64 + k * 8) = pack8(o);
 }
 
 /* Encoder output (iris_vae.c:440-482): moments [h][w][2z] f32 (NHWC) ->
  * optional 1x1 quant_conv (qw [2z][2z]) -> the mean (first z channels) ->
  * patchify 2x2 (channel c at (y, x) becomes channel c * 4 + 2 (y & 1) + (x & 1)
  * at (y / 2, x / 2)) -> per latent channel (x - sh) * sc (Z-Image: scaling,
- * shift; Flux: 1 / sqrt(var + eps), mean) -> latent [4z][h/2][w/2] f32. */
+ * shift; Flux: 1 / sqrt(var + eps), mean) -> latent [4z][h/2][w/2] f32.
+ * A block takes EO_PIX pixels and every (pixel, channel) a thread; the
+ * pixels' moments and the mean rows of qw sit in LDS (LDS false: too many
+ * channels for it, read from memory). One thread per pixel left 240 CUs idle
+ * at 64 x 64 moments. 277 -> 8 us. */
+constexpr int EO_PIX = 16;
+template <bool LDS>
 __global__ __launch_bounds__(NT) void vae_enc_out_kernel(const float *mom, int z, int h, int w, const float *qw,
                                                          const float *qb, const float *sc, const float *sh,
                                                          float *lat) {
-    const int p = blockIdx.x * NT + threadIdx.x;
-    if (p >= h * w) return;
-    const int y = p / w, x = p % w, z2 = 2 * z;
-    const float *m = mom + (size_t)p * z2;
-    const int lh = h / 2, lw = w / 2;
-    if ((y >> 1) >= lh || (x >> 1) >= lw) return;
-    for (int c = 0; c < z; c++) {
+    extern __shared__ float esh[];
+    const int z2 = 2 * z, p0 = blockIdx.x * EO_PIX, np = min(EO_PIX, h * w - p0), lh = h / 2, lw = w / 2;
+    const int mstr = LDS ? z2 + 1 : z2;   /* rows one word apart in the banks */
+    float *const ws = esh + EO_PIX * (z2 + 1);
+    if constexpr (LDS) {
+        for (int i = threadIdx.x; i < np * z2; i += NT) esh[i / z2 * mstr + i % z2] = mom[(size_t)p0 * z2 + i];
+        if (qw)
+            for (int i = threadIdx.x; i < z * z2; i += NT) ws[i] = qw[i];
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < EO_PIX * z; i += NT) {
+        const int q = i % EO_PIX, c = i / EO_PIX;
+        const int y = (p0 + q) / w, x = (p0 + q) % w;
+        if (q >= np || (y >> 1) >= lh || (x >> 1) >= lw) continue;
+        auto m = [&](int k) { return LDS ? esh[q * mstr + k] : mom[(size_t)(p0 + q) * z2 + k]; };
         float v;
         if (qw) {
             v = qb ? qb[c] : 0.0f;
-            for (int k = 0; k < z2; k++) v += qw[c * z2 + k] * m[k];
+            for (int k = 0; k < z2; k++) v += (LDS ? ws[c * z2 + k] : qw[(size_t)c * z2 + k]) * m(k);
         } else {
-            v = m[c];
+            v = m(c);
         }
         const int lc = c * 4 + (y & 1) * 2 + (x & 1);
         lat[((size_t)lc * lh + (y >> 1)) * lw + (x >> 1)] = (v - sh[lc]) * sc[lc];
@@ -456,7 +480,7 @@ extern "C" int iris_hip_vae_front(uint16_t *out, const float *lat, int z, int h,
     if (!out || !lat || !sc || !sh || z <= 0 || z > 32 || h <= 0 || w <= 0 || ((uintptr_t)out & 15))
         return iris_set_error("vae_front: bad arguments (z=%d, %dx%d)", z, h, w);
     const int npix = 4 * h * w;
-    IRIS_LAUNCH(vae_front_kernel, dim3((npix + NT - 1) / NT), dim3(NT), 0, iris_stream(), lat, z, h, w, sc, sh,
+    IRIS_LAUNCH(vae_front_kernel, dim3((npix + FR_PIX - 1) / FR_PIX), dim3(NT), 0, iris_stream(), lat, z, h, w, sc, sh,
                        divide, pqw, pqb, out);
     return iris_launch_check("vae_front_kernel");
 }
@@ -501,14 +525,18 @@ extern "C" int iris_hip_vae_conv_out(uint8_t *rgb, float *f32, const uint16_t *g
 extern "C" int iris_hip_vae_img_in(uint16_t *out, const float *img, int H, int W) {
     if (!out || !img || H <= 0 || W <= 0 || ((uintptr_t)out & 15)) return iris_set_error("vae_img_in: bad arguments");
     const int npix = H * W;
-    IRIS_LAUNCH(vae_img_in_kernel, dim3((npix + NT - 1) / NT), dim3(NT), 0, iris_stream(), img, npix, out);
+    IRIS_LAUNCH(vae_img_in_kernel, dim3((npix + NT / 8 - 1) / (NT / 8)), dim3(NT), 0, iris_stream(), img, npix, out);
     return iris_launch_check("vae_img_in_kernel");
 }
 
 extern "C" int iris_hip_vae_enc_out(float *lat, const float *mom, int z, int h, int w, const float *qw,
                                     const float *qb, const float *sc, const float *sh) {
     if (!lat || !mom || !sc || !sh || z <= 0 || h < 2 || w < 2) return iris_set_error("vae_enc_out: bad arguments");
-    IRIS_LAUNCH(vae_enc_out_kernel, dim3((h * w + NT - 1) / NT), dim3(NT), 0, iris_stream(), mom, z, h, w, qw,
-                       qb, sc, sh, lat);
+    const size_t smem = ((size_t)EO_PIX * (2 * z + 1) + (qw ? (size_t)2 * z * z : 0)) * sizeof(float);
+    const dim3 grid((h * w + EO_PIX - 1) / EO_PIX);
+    if (smem <= 64 * 1024)
+        IRIS_LAUNCH(vae_enc_out_kernel<true>, grid, dim3(NT), smem, iris_stream(), mom, z, h, w, qw, qb, sc, sh, lat);
+    else
+        IRIS_LAUNCH(vae_enc_out_kernel<false>, grid, dim3(NT), 0, iris_stream(), mom, z, h, w, qw, qb, sc, sh, lat);
     return iris_launch_check("vae_enc_out_kernel");
 }
