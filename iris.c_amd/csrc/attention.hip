@@ -68,6 +68,14 @@
  * descriptors; K's range ends at its last valid row so rows past the end read
  * as zero.
  *
+ * Launches of few units take blocks of 4 waves and 128 queries (NWV = 4): one
+ * wave per SIMD, the softmax of a tile under the QK products of the next.
+ *
+ * The Q prologue is VALU work (4 clocks an instruction per wave), so it uses
+ * the hardware reciprocal square root and bf16 conversion and picks the
+ * weight set once per wave: 3 to 4 us less per round of blocks (768 queries,
+ * 72 units 28.1 -> 25.0 us; 4608, two rounds, 252.8 -> 247.1 us).
+ *
  * Blocks are ordered head-major and mapped XCD-major (block b runs on XCD
  * b % 8 and takes a contiguous range of the work list), so the query blocks
  * of one head share its K and V in one XCD's L2.
@@ -87,11 +95,11 @@ enum { F_FUSEQ = 1, F_CAUSAL = 2, F_BIAS = 4, F_SPLIT = 8 };
 
 /* LDS of one block: two K stages, two V^T stages and, with the Q prologue,
  * each wave's 32 normalised, rotated rows after them */
-template <int FEAT> struct AttnLds {
+template <int FEAT, int NWV> struct AttnLds {
     static constexpr bool V16 = !(FEAT & F_SPLIT); /* V^T read as 16-byte chunks */
     static constexpr int VSTR = V16 ? KB + 8 : KB + 4, VS_ELEMS = HD * VSTR;
     static constexpr int QS_OFF = 2 * KS_ELEMS + 2 * VS_ELEMS;
-    static constexpr size_t BYTES = (size_t)QS_OFF * 2 + ((FEAT & F_FUSEQ) ? (size_t)NW * 32 * KSTR * 2 : 0);
+    static constexpr size_t BYTES = (size_t)QS_OFF * 2 + ((FEAT & F_FUSEQ) ? (size_t)NWV * 32 * KSTR * 2 : 0);
 };
 
 /* Balanced schedule (F_SPLIT): the nkt key tiles of all units (query block,
@@ -129,12 +137,16 @@ struct AttnSeg {
 /* s_waitcnt immediate: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8 */
 constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8); }
 
-template <int FEAT>
+template <int FEAT, int NWV>
 __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float scale_log2, int nqb, const int L,
                                              const int t0, int tn, const AttnSplit &sp, const AttnSeg sg) {
     constexpr bool FUSEQ = FEAT & F_FUSEQ, CAUSAL = FEAT & F_CAUSAL, BIAS = FEAT & F_BIAS;
-    constexpr bool V16 = AttnLds<FEAT>::V16;
-    constexpr int VSTR = AttnLds<FEAT>::VSTR, VS_ELEMS = AttnLds<FEAT>::VS_ELEMS, QS_OFF = AttnLds<FEAT>::QS_OFF;
+    using Lds = AttnLds<FEAT, NWV>;
+    constexpr bool V16 = Lds::V16;
+    constexpr int VSTR = Lds::VSTR, VS_ELEMS = Lds::VS_ELEMS, QS_OFF = Lds::QS_OFF;
+    /* NWV = 8 waves: 256 queries, two wave groups; 4: 128 queries, one. A
+     * group's 256 threads stage its share of a tile in CH chunks each */
+    constexpr int NTB = NWV * 64, QBB = NWV * QW, CH = NWV == 8 ? 2 : 4;
     extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
 #define KBUF(b) (smem + (b) * KS_ELEMS)
 #define VBUF(b) (smem + 2 * KS_ELEMS + (b) * VS_ELEMS)
@@ -144,7 +156,7 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
     const int kv_head = a.kv_group > 1 ? head / a.kv_group : head;
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int grp = wave >> 2, gt = tid & 255;
+    const int grp = NWV == 8 ? wave >> 2 : 0, gt = tid & 255;
     const uint16_t *Q = a.q + (size_t)bz * a.q_bstride + head * HD;
     const uint16_t *K = a.k + (size_t)bz * a.k_bstride + kv_head * HD;
     const uint16_t *VT = a.vt + (size_t)bz * a.vt_bstride + (size_t)kv_head * HD * a.ld_vt;
@@ -153,8 +165,8 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
     /* the segment's key tiles, t0 .. t0 + nkt - 1 (tn < 0: all; causal: the
      * block's last query needs keys up to its own index) */
     const int nkt = tn >= 0 ? tn
-                            : CAUSAL ? (min(sk, min(sq, (qblk + 1) * QB)) + KB - 1) / KB : (sk + KB - 1) / KB;
-    const int wave_q0 = qblk * QB + wave * QW;
+                            : CAUSAL ? (min(sk, min(sq, (qblk + 1) * QBB)) + KB - 1) / KB : (sk + KB - 1) / KB;
+    const int wave_q0 = qblk * QBB + wave * QW;
     const int q_row = wave_q0 + lr;
 
     /* Every tile offset goes into the VGPR offset, which the buffer range check
@@ -164,8 +176,8 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
     const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void *)VT, (short)0, (int)((size_t)HD * a.ld_vt * 2), 0x00020000);
 
-    /* this group's half of a tile: K rows 32 grp + gt/16 (+ 16), chunk gt % 16;
-     * V^T d rows 64 grp + gt/8 (+ 32), chunk gt % 8 */
+    /* this group's share of a tile: K rows 32 grp + gt/16 (+ 16 i), chunk gt % 16;
+     * V^T d rows 64 grp + gt/8 (+ 32 i), chunk gt % 8 */
     const int kh_off = ((32 * grp + (gt >> 4)) * a.ld_k + (gt & 15) * 8) * 2;
     const int vh_off = ((64 * grp + (gt >> 3)) * a.ld_vt + (gt & 7) * 8) * 2;
     uint16_t *const kh_dst = smem + (32 * grp + (gt >> 4)) * KSTR + (gt & 15) * 8;
@@ -174,38 +186,39 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
      * 4 (c % 2), its last 4 to 8 + 4 (c % 2) of the block */
     uint16_t *const vh_dst = smem + 2 * KS_ELEMS + (64 * grp + (gt >> 3)) * VSTR +
                              (V16 ? 16 * ((gt & 7) >> 1) + 4 * (gt & 1) : 8 * (gt & 7));
-    uint4 rk[2], rv[2];
+    uint4 rk[CH], rv[CH];
     auto load_k = [&](int kt) {
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int i = 0; i < CH; i++)
             rk[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                                   k_rsrc, kh_off + ((t0 + kt) * KB + 16 * i) * a.ld_k * 2, 0, 0));
     };
     auto load_v = [&](int kt) {
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int i = 0; i < CH; i++)
             rv[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                                   v_rsrc, vh_off + (32 * i * a.ld_vt + (t0 + kt) * KB) * 2, 0, 0));
     };
     auto store_k = [&](int stage) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) *(uint4 *)(kh_dst + stage * KS_ELEMS + 16 * i * KSTR) = rk[i];
+        for (int i = 0; i < CH; i++) *(uint4 *)(kh_dst + stage * KS_ELEMS + 16 * i * KSTR) = rk[i];
     };
     auto store_v = [&](int stage) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < CH; i++) {
             uint16_t *d = vh_dst + stage * VS_ELEMS + 32 * i * VSTR;
             *(uint2 *)d = make_uint2(rv[i].x, rv[i].y);
             *(uint2 *)(d + (V16 ? 8 : 4)) = make_uint2(rv[i].z, rv[i].w);
         }
     };
-    /* the whole K(0) tile: rows tid/16 and + 32, chunk tid % 16 */
-    uint4 k0r[2];
+    /* the whole K(0) tile: rows tid/16 (+ NTB/16 i), chunk tid % 16 */
+    uint4 k0r[CH];
     {
         const int k_off = ((tid >> 4) * a.ld_k + (tid & 15) * 8) * 2 + t0 * KB * a.ld_k * 2;
-        k0r[0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, k_off, 0, 0));
-        k0r[1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, k_off + 32 * a.ld_k * 2,
-                                                                                  0, 0));
+#pragma unroll
+        for (int i = 0; i < CH; i++)
+            k0r[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                   k_rsrc, k_off + i * (NTB / 16) * a.ld_k * 2, 0, 0));
     }
     /* Q loads next, so that their latency and K(0)'s overlap: the fragments
      * (B operand: lane holds query lr of the wave's 32, d = ds*16 + lg*8 ..
@@ -264,8 +277,8 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
     load_v(0);
     {
         uint16_t *kd = KBUF(0) + (tid >> 4) * KSTR + (tid & 15) * 8;
-        *(uint4 *)kd = k0r[0];
-        *(uint4 *)(kd + 32 * KSTR) = k0r[1];
+#pragma unroll
+        for (int i = 0; i < CH; i++) *(uint4 *)(kd + i * (NTB / 16) * KSTR) = k0r[i];
     }
 
     /* Q prologue: the raw rows loaded above, with the arithmetic of the K
@@ -273,6 +286,10 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
      * back in the B-operand layout */
     auto q_prologue = [&]() {
         uint16_t *qs = smem + QS_OFF + wave * 32 * KSTR;
+        /* the wave's rows take one weight set, but for the wave that holds
+         * the line between the two (row order: set A first) */
+        const bool mixed = wave_q0 < a.qn_split && wave_q0 + QW > a.qn_split;
+        float4 ww0 = wave_q0 < a.qn_split ? wa0 : wb0, ww1 = wave_q0 < a.qn_split ? wa1 : wb1;
 #pragma unroll
         for (int pass = 0; pass < 8; pass++) {
             const int rw = pass * 4 + rl, row = wave_q0 + rw;
@@ -280,18 +297,17 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
 #pragma unroll
             for (int j = 0; j < 8; j++) { x[j] = bf2f(raw[pass][j]); ss += x[j] * x[j]; }
             ss = row16_sum(ss);
-            const float inv = 1.0f / sqrtf(ss / 128.0f + a.qn_eps);
-            const bool sa = row < a.qn_split;
-            const float ww[8] = {sa ? wa0.x : wb0.x, sa ? wa0.y : wb0.y, sa ? wa0.z : wb0.z, sa ? wa0.w : wb0.w,
-                                 sa ? wa1.x : wb1.x, sa ? wa1.y : wb1.y, sa ? wa1.z : wb1.z, sa ? wa1.w : wb1.w};
+            const float inv = __builtin_amdgcn_rsqf(ss * (1.0f / 128.0f) + a.qn_eps);
+            if (mixed && row >= a.qn_split) { ww0 = wb0; ww1 = wb1; }
+            const float ww[8] = {ww0.x, ww0.y, ww0.z, ww0.w, ww1.x, ww1.y, ww1.z, ww1.w};
             const float c[4] = {c4[pass].x, c4[pass].y, c4[pass].z, c4[pass].w};
             const float sn[4] = {s4[pass].x, s4[pass].y, s4[pass].z, s4[pass].w};
             u16x8 out;
 #pragma unroll
             for (int j = 0; j < 8; j += 2) {
                 const float x0 = x[j] * inv * ww[j], x1 = x[j + 1] * inv * ww[j + 1];
-                out[j] = f2bf(x0 * c[j >> 1] - x1 * sn[j >> 1]);
-                out[j + 1] = f2bf(x1 * c[j >> 1] + x0 * sn[j >> 1]);
+                out[j] = f2bf_hw(x0 * c[j >> 1] - x1 * sn[j >> 1]);
+                out[j + 1] = f2bf_hw(x1 * c[j >> 1] + x0 * sn[j >> 1]);
             }
             *(u16x8 *)(qs + rw * KSTR + d0) = out;
         }
@@ -309,7 +325,7 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
     /* running max of the lane's query column (same in both lanes of the column)
      * and this lane's partial row sum over its half of each tile's keys */
     float m_run = -1e30f, l_run = 0.0f;
-    f32x16 s[2];
+    f32x16 s[2], s2[2];   /* s2: NWV = 4, the next tile's */
     bf16x8 pf[4];
 
     auto bar = [&]() {
@@ -341,7 +357,7 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
         }
     };
     /* S^T of the tile in K stage kst */
-    auto qk = [&](int kst) {
+    auto qk = [&](int kst, f32x16 (&s)[2]) {
         const uint16_t *kb = KBUF(kst);
 #pragma unroll
         for (int ks = 0; ks < 2; ks++)
@@ -368,9 +384,9 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
         __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
     };
 
-    /* V phase of tile t: masks, max, lazy rescale, P = exp2(S - m) as bf16
-     * B-operand fragments, row sums */
-    auto v_phase = [&](int t) {
+    /* V phase of tile t: masks, max, lazy rescale, then P = exp2(S - m) as
+     * bf16 B-operand fragments and row sums */
+    auto v_max = [&](int t, f32x16 (&s)[2]) {
         const int k0 = (t0 + t) * KB;
         const bool full = k0 + KB <= sk && ((k0 >= a.kv_lo0 && k0 + KB <= a.kv_hi0) ||
                                             (k0 >= a.kv_lo1 && k0 + KB <= a.kv_hi1)) &&
@@ -417,6 +433,8 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
 #pragma unroll
                 for (int r = 0; r < 16; r++) o[dsub][r] *= alpha;
         }
+    };
+    auto v_exp = [&](const f32x16 (&s)[2]) {
         float rs = 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -432,18 +450,72 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
         l_run += rs;
     };
 
+    if constexpr (NWV == 4) {
+        /* One wave per SIMD: the softmax of tile t runs under the QK products
+         * of tile t+1 in the same wave (S of both in registers), then the
+         * products PV(t), with K(t+2) and V(t+1) staged and the loads of
+         * K(t+3) and V(t+2) issued among them; one barrier per tile (the
+         * stages written in iteration t were last read in t-1). */
+        auto iter = [&](int t, f32x16 (&cur)[2], f32x16 (&nxt)[2]) {
+            v_max(t, cur);
+            __builtin_amdgcn_sched_barrier(0);
+            qk((t + 1) & 1, nxt);
+            v_exp(cur);
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (i < 12) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+                __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            store_k(t & 1);
+            store_v((t + 1) & 1);
+            load_k(min(t + 3, nkt - 1));
+            load_v(min(t + 2, nkt - 1));
+            pv(t & 1);
+            interleave(16);
+            bar();
+        };
+        bar();   /* K(0) staged */
+        if (nkt > 1) store_k(1);
+        store_v(0);
+        load_k(min(2, nkt - 1));
+        if (nkt > 1) load_v(1);
+        qk(0, s);
+        bar();
+        int t = 0;
+        for (; t + 2 < nkt; t += 2) {
+            iter(t, s, s2);
+            iter(t + 1, s2, s);
+        }
+        if (t + 1 < nkt) {
+            iter(t, s, s2);
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) s[ks] = s2[ks];
+        }
+        v_max(nkt - 1, s);
+        v_exp(s);
+        pv((nkt - 1) & 1);
+        bar();
+    } else {
     /* In its M(t) phase a group stages K(t+1) and V(t) from registers, loads
      * K(t+2) and V(t+1) (indices clamped to the last tile near the end: a
      * clamped K lands in a stage nothing reads again), then runs PV(t-1) and
      * QK(t). Group 0: M(0) V(0) M(1) ... V(nkt-1) M(nkt); group 1 one phase
      * later. Both execute 2 nkt + 3 barriers. */
+    auto v_phase = [&](int t) {
+        v_max(t, s);
+        v_exp(s);
+    };
     bar();   /* K(0) staged */
     if (grp) bar();
     if (nkt > 1) store_k(1);
     store_v(0);
     load_k(min(2, nkt - 1));
     if (nkt > 1) load_v(1);
-    qk(0);
+    qk(0, s);
     bar();
     v_phase(0);
     bar();
@@ -453,7 +525,7 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
         load_k(min(t + 2, nkt - 1));
         load_v(min(t + 1, nkt - 1));
         pv((t - 1) & 1);
-        qk(t & 1);
+        qk(t & 1, s);
         interleave(32);
         bar();
         v_phase(t);
@@ -462,6 +534,7 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
     pv((nkt - 1) & 1);
     bar();
     if (!grp) bar();
+    }
 
     if ((FEAT & F_SPLIT) && sg.part) {
         /* a piece of the unit: store o, m, l at system coherence (written
@@ -525,7 +598,7 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
          * 256 rows of 128 + 8 elements, then 16-byte chunks of whole rows, so a
          * store instruction writes 4 full rows instead of 16-byte pieces of 32 */
         constexpr int OSTR = HD + 8;
-        static_assert(QB * OSTR <= QS_OFF, "the O tile fits the K and V stages");
+        static_assert(QBB * OSTR <= QS_OFF, "the O tile fits the K and V stages");
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
         uint16_t *const orow = smem + (wave * QW + lr) * OSTR;
 #pragma unroll
@@ -534,15 +607,15 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
             for (int rb = 0; rb < 4; rb++) {
                 u16x4 v;
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = f2bf(o[dsub][rb * 4 + e] * inv);
+                for (int e = 0; e < 4; e++) v[e] = f2bf_hw(o[dsub][rb * 4 + e] * inv);
                 *(u16x4 *)(orow + dsub * 32 + rb * 8 + lg * 4) = v;
             }
         __syncthreads();
-        uint16_t *const Ob = O + (size_t)(qblk * QB) * a.ld_o;
-        const int nrow = min(QB, sq - qblk * QB);
+        uint16_t *const Ob = O + (size_t)(qblk * QBB) * a.ld_o;
+        const int nrow = min(QBB, sq - qblk * QBB);
 #pragma unroll
-        for (int i = 0; i < QB * (HD / 8) / NT; i++) {
-            const int c = tid + NT * i, row = c >> 4, ch = c & 15;
+        for (int i = 0; i < QBB * (HD / 8) / NTB; i++) {
+            const int c = tid + NTB * i, row = c >> 4, ch = c & 15;
             if (row < nrow) *(uint4 *)(Ob + (size_t)row * a.ld_o + ch * 8) = *(const uint4 *)(smem + row * OSTR + ch * 8);
         }
     } else if (q_row < sq) {
@@ -554,7 +627,7 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
                 const int d = dsub * 32 + rb * 8 + lg * 4;
                 u16x4 v;
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = f2bf(o[dsub][rb * 4 + e] * inv);
+                for (int e = 0; e < 4; e++) v[e] = f2bf_hw(o[dsub][rb * 4 + e] * inv);
                 *(u16x4 *)(O + (size_t)q_row * a.ld_o + d) = v;
             }
     }
@@ -562,30 +635,30 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
 #undef VBUF
 }
 
-template <int FEAT>
-__global__ __launch_bounds__(NT) void flash_attn_kernel(const iris_attn_args_t a, float scale_log2, int nqb,
+template <int FEAT, int NWV = NW>
+__global__ __launch_bounds__(NWV * 64, 2) void flash_attn_kernel(const iris_attn_args_t a, float scale_log2, int nqb,
                                                         int per_xcd, int total, const AttnSplit sp) {
     if constexpr (!(FEAT & F_SPLIT)) {
         const int L = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
         if (L >= total) return;
-        attn_segment<FEAT>(a, scale_log2, nqb, L, 0, -1, sp, AttnSeg{0, 0, 0});
+        attn_segment<FEAT, NWV>(a, scale_log2, nqb, L, 0, -1, sp, AttnSeg{0, 0, 0});
     } else {
         const int s = (blockIdx.x & 7) * sp.bpx + (blockIdx.x >> 3), end = split_start(sp, s + 1);
         for (int it = split_start(sp, s), first = 1; it < end; first = 0) {
             const int unit = it / sp.nkt, t0 = it - unit * sp.nkt, tn = min(sp.nkt - t0, end - it);
             if (!first) __syncthreads();   /* the previous segment's LDS reads are done */
-            attn_segment<FEAT>(a, scale_log2, nqb, unit, t0, tn, sp, AttnSeg{tn != sp.nkt, s, first});
+            attn_segment<FEAT, NWV>(a, scale_log2, nqb, unit, t0, tn, sp, AttnSeg{tn != sp.nkt, s, first});
             it += tn;
         }
     }
 }
 
-template <int FEAT>
+template <int FEAT, int NWV = NW>
 int launch(const iris_attn_args_t *a, float scale_log2, int nqb, int per_xcd, int total, const AttnSplit &sp) {
-    constexpr size_t smem = AttnLds<FEAT>::BYTES;
+    constexpr size_t smem = AttnLds<FEAT, NWV>::BYTES;
     static bool attr_set = false;
     if (!attr_set) {
-        if (iris_check(hipFuncSetAttribute((const void *)flash_attn_kernel<FEAT>,
+        if (iris_check(hipFuncSetAttribute((const void *)flash_attn_kernel<FEAT, NWV>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem),
                        "attention smem attribute"))
             return -1;
@@ -597,8 +670,11 @@ int launch(const iris_attn_args_t *a, float scale_log2, int nqb, int per_xcd, in
         "flash_attn_kernel<8>",  "flash_attn_kernel<9>",  "flash_attn_kernel<10>", "flash_attn_kernel<11>",
         "flash_attn_kernel<12>", "flash_attn_kernel<13>", "flash_attn_kernel<14>", "flash_attn_kernel<15>"};
     const unsigned grid = (FEAT & F_SPLIT) ? 8u * sp.bpx : 8u * per_xcd;
-    const int prof = iris_prof_begin(name[FEAT & 15], grid);
-    hipLaunchKernelGGL(flash_attn_kernel<FEAT>, dim3(grid), dim3(NT), smem, iris_stream(), *a, scale_log2, nqb, per_xcd,
+    static const char *const name4[8] = {"flash_attn_kernel<0, 4>", "flash_attn_kernel<1, 4>", "flash_attn_kernel<2, 4>",
+                                         "flash_attn_kernel<3, 4>", "flash_attn_kernel<4, 4>", "flash_attn_kernel<5, 4>",
+                                         "flash_attn_kernel<6, 4>", "flash_attn_kernel<7, 4>"};
+    const int prof = iris_prof_begin(NWV == 4 ? name4[FEAT & 7] : name[FEAT & 15], grid);
+    hipLaunchKernelGGL((flash_attn_kernel<FEAT, NWV>), dim3(grid), dim3(NWV * 64), smem, iris_stream(), *a, scale_log2, nqb, per_xcd,
                        total, sp);
     iris_prof_end(prof);
     return iris_launch_check("flash_attn_kernel");
@@ -656,6 +732,26 @@ extern "C" int iris_hip_attention(const iris_attn_args_t *a) {
             sp.ws = (float *)((char *)a->ws + SPLIT_CNT_BYTES);
             sp.slots = 2 * cus;
             feat |= F_SPLIT;
+        }
+    }
+    /* 128 queries per block (4 waves) where those blocks still fit one round:
+     * twice the CUs at work, and half the prologue per CU. Same bits. Measured,
+     * us, 8 waves -> 4 (24 heads, keys = queries): 768 25.0 -> 20.7, 1024 31.4
+     * -> 26.6, 1280 37.1 -> 31.6; 32 heads causal: 37 11.1 -> 7.9, 512 26.0 ->
+     * 17.9. Past one round the second one costs more: 1536 (288 blocks) 42.0
+     * -> 65.6, and at 4608 the two groups' overlap wins, 247 -> 345. */
+    const int nqb4 = (a->sq + 4 * QW - 1) / (4 * QW);
+    const long long total4 = (long long)nqb4 * a->heads * a->batch;
+    if (total4 <= cus) {
+        const int px = (int)((total4 + 7) / 8), n = (int)total4;
+        switch (feat) {
+        case 0: return launch<0, 4>(a, scale_log2, nqb4, px, n, sp);
+        case F_FUSEQ: return launch<F_FUSEQ, 4>(a, scale_log2, nqb4, px, n, sp);
+        case F_CAUSAL: return launch<F_CAUSAL, 4>(a, scale_log2, nqb4, px, n, sp);
+        case F_FUSEQ | F_CAUSAL: return launch<F_FUSEQ | F_CAUSAL, 4>(a, scale_log2, nqb4, px, n, sp);
+        case F_BIAS: return launch<F_BIAS, 4>(a, scale_log2, nqb4, px, n, sp);
+        case F_FUSEQ | F_BIAS: return launch<F_FUSEQ | F_BIAS, 4>(a, scale_log2, nqb4, px, n, sp);
+        default: break;
         }
     }
     switch (feat) {
