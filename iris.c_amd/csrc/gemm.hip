@@ -1629,7 +1629,12 @@ extern "C" int iris_hip_softmax_scores(const uint16_t *q, int ld_q, const uint16
     return iris_launch_check("gemm_bf16_kernel<5> (probabilities)");
 }
 
-extern "C" int iris_hip_conv3x3(const iris_conv3x3_t *c) {
+namespace {
+
+/* checks a convolution and fills what its kernels need for tiles of bnt
+ * output channels (bnt 0: 128 for at most 128 channels -- the decoder's
+ * full-resolution convolutions -- else 256; the same additions per element) */
+int conv_params(const iris_conv3x3_t *c, int bnt, GemmParams &P) {
     if (!c || !c->in || !c->wt || !c->out) return iris_set_error("conv3x3: null operand");
     if (c->cin < 64 || c->cin > 8192 || (c->cin & (c->cin - 1)))
         return iris_set_error("conv3x3: cin=%d must be a power of two in 64..8192", c->cin);
@@ -1655,15 +1660,12 @@ extern "C" int iris_hip_conv3x3(const iris_conv3x3_t *c) {
     p.lda = p.ldw = p.K;
     p.ldo = c->ldo;
     p.epi = c->epi;
+    memset(&P, 0, sizeof(P));
+    P.p[0] = p;
     if (p.N <= 0) return 0;
     if (check_problem(p)) return -1;
-    GemmParams P;
-    memset(&P, 0, sizeof(P));
     P.nprob = 1;
-    P.p[0] = p;
-    /* 128-wide tiles for at most 128 output channels (the decoder's
-     * full-resolution convolutions): same per-element accumulation order */
-    const int bnt = p.N <= 128 ? 128 : BN;
+    if (!bnt) bnt = p.N <= 128 ? 128 : BN;
     P.tiles_m[0] = (p.M + BM - 1) / BM;
     P.tiles_n[0] = (p.N + bnt - 1) / bnt;
     P.conv_h = c->H;
@@ -1681,6 +1683,17 @@ extern "C" int iris_hip_conv3x3(const iris_conv3x3_t *c) {
         P.gn_part = c->gn_part;
         P.gn_groups = G;
     }
+    return 0;
+}
+
+}  // namespace
+
+extern "C" int iris_hip_conv3x3(const iris_conv3x3_t *c) {
+    GemmParams P;
+    if (conv_params(c, 0, P)) return -1;
+    const iris_gemm_problem_t &p = P.p[0];
+    if (p.N <= 0) return 0;
+    const int bnt = p.N <= 128 ? 128 : BN;
     int chunks = 1;
     long long stride = 0;
     P.chunks[0] = 1;
@@ -1713,4 +1726,346 @@ extern "C" int iris_hip_conv3x3(const iris_conv3x3_t *c) {
     if (chunks == 1) return 0;
     float *rws = c->ws;
     return launch_reduce(&p, &rws, &stride, &chunks, 1);
+}
+
+namespace {
+
+/* 3x3 convolution, stride 1 (UP: the input read through a nearest 2x
+ * upsample), one 16 x 16 pixel tile x 128 output channels per block. The
+ * implicit GEMM above loads an input pixel from L2 once per tap: 48 KiB per
+ * 64-wide K step of a 256 x 128 tile, more than a CU gets in the time of the
+ * step's products. Here the tile's pixels and their halo (18 x 18, or 10 x 10
+ * before the upsample) are staged once per 64 channels and all nine taps read
+ * their fragments from that patch; only the weights (16 KiB per step) stream:
+ * 189 KiB per 64 channels instead of 432. The tile then leaves through LDS,
+ * the residual of IRIS_EPI_ADD in flight while it is staged. Measured against
+ * the implicit GEMM, us: 1024 x 1024, 128 -> 128 with the residual 498 -> 367
+ * (f32 stream in and out: 210 of it), bf16 out 342 -> 311, 256 -> 128 619 ->
+ * 497; 512 x 512, 512 -> 256 467 -> 429 (1.44 PFLOP/s); 256 x 256 x 512
+ * upsampled 219 -> 196 (1.58); 128 x 128, 512 -> 512 80.5 -> 53.8. The direct
+ * stores of the accumulators took 614 where it takes 367: 64-byte pieces,
+ * behind a load each.
+ *
+ * 8 waves as in gemm_ring_kernel: waves 0..3 compute (2x2, wave tile 8 pixel
+ * rows x 64 channels), waves 4..7 load, one barrier per K step (a tap of a
+ * 64-channel chunk; taps within chunks). Weights go through 4 stages. The
+ * patch has two buffers: chunk c+1's is loaded in the first AL steps of chunk
+ * c, and it is complete when step 8 of chunk c waits for the weights of the
+ * next step, which each step issues after its patch loads (loads of a wave
+ * complete in order).
+ *
+ * LDS patch pixel (r, c) is row r PW + c of 128 bytes, its 16-byte chunk k
+ * stored at k ^ ((c / 2) mod 8): PW is even, so 16 neighbouring columns of a
+ * row lie in 16 distinct bank groups, and the swizzle depends on the lane
+ * only: every fragment is one of six lane addresses plus a constant. */
+struct ConvParams {
+    const uint16_t *in, *wt;
+    void *out;
+    const float *bias;
+    int H, W, cin, cout, ldo, epi;
+    int tx, tn, tiles, total, per_xcd;   /* tile columns, 128-channel tiles, blocks of a split, of all */
+    int cps;                             /* 64-channel chunks per split of K */
+    float *ws;                           /* f32 partials of the splits, ws_stride apart; NULL: one split */
+    long long ws_stride;
+    unsigned in_bytes;
+    double *gn_part;
+    int gn_groups;
+};
+
+template <bool UP>
+__global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) {
+    constexpr int PW = UP ? 10 : 18, NPX = PW * PW, SLOTS = (NPX + 7) / 8, AL = (SLOTS + 7) / 8;
+    constexpr int A_BYTES = SLOTS * 1024, W_BYTES = 128 * BK * 2, NSW = 4, FM_ = 8, FN_ = 4;
+    extern __shared__ __attribute__((aligned(16))) char sm[];
+    __shared__ float gnl[16][32][2];
+    const int L = (blockIdx.x & 7) * P.per_xcd + (blockIdx.x >> 3);
+    if (L >= P.total) return;
+    /* scalar registers for what the buffer resources and addresses are made of */
+    const int split = __builtin_amdgcn_readfirstlane(L / P.tiles), Ls = L - split * P.tiles;
+    const int tile = __builtin_amdgcn_readfirstlane(Ls / P.tn), ty = __builtin_amdgcn_readfirstlane(tile / P.tx);
+    const int n0 = (Ls - tile * P.tn) * 128, y0 = ty * 16, x0 = (tile - ty * P.tx) * 16;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c0 = split * P.cps, chunks = min(P.cps, P.cin / BK - c0);   /* this block's 64-channel chunks */
+    char *const wring = sm + 2 * A_BYTES;
+    const bool gn = P.gn_part != nullptr;
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (wave >= 4) {
+        const int lw = wave & 3, drow = lane >> 3, dch = lane & 7;
+        const __amdgpu_buffer_rsrc_t a_rsrc =
+            __builtin_amdgcn_make_buffer_rsrc((void *)P.in, (short)0, (int)P.in_bytes, 0x00020000);
+        const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(P.wt + (size_t)n0 * 9 * P.cin), (short)0, min(128, P.cout - n0) * 9 * P.cin * 2, 0x00020000);
+        /* patch slot j holds patch pixels 8j .. 8j+7; this wave's are
+         * 8s + 2 lw + i of step s (the last slot again past the end). Pixels
+         * outside the image, and past the patch, read as zero: an offset past
+         * the end of the buffer */
+        const int hin = UP ? P.H / 2 : P.H, win = UP ? P.W / 2 : P.W;
+        const int py0 = (UP ? y0 / 2 : y0) - 1, px0 = (UP ? x0 / 2 : x0) - 1;
+        int a_off[12];   /* 2 AL of them */
+#pragma unroll
+        for (int i = 0; i < 2 * AL; i++) {
+            const int px = min((i >> 1) * 8 + lw * 2 + (i & 1), SLOTS - 1) * 8 + drow;
+            const int r = px / PW, c = px - r * PW, gy = py0 + r, gx = px0 + c;
+            const bool ok = px < NPX && (unsigned)gy < (unsigned)hin && (unsigned)gx < (unsigned)win;
+            a_off[i] = ok ? (gy * win + gx) * P.cin * 2 + ((dch ^ ((c >> 1) & 7)) << 4) : (int)0x80000000u;
+        }
+        int w_off[2];
+#pragma unroll
+        for (int par = 0; par < 2; par++)
+            w_off[par] = (lw * 32 + drow) * 9 * P.cin * 2 + ((dch ^ ((4 * par + (drow >> 1)) & 7)) << 4);
+        const int w_step = 8 * 9 * P.cin * 2;
+        auto dma_a = [&](int chunk, int i) {
+            const int slot = min((i >> 1) * 8 + lw * 2 + (i & 1), SLOTS - 1);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                a_rsrc, (lds_void *)(sm + (chunk & 1) * A_BYTES + slot * 1024), 16, a_off[i],
+                (c0 + min(chunk, chunks - 1)) * (BK * 2), 0, 0);
+        };
+        auto dma_w = [&](int stage, int chunk, int tap) {
+            const int soff = (tap * P.cin + (c0 + chunk) * BK) * 2;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(wring + stage * W_BYTES + (lw * 4 + i) * 1024),
+                                                         16, w_off[i & 1] + i * w_step, soff, 0, 0);
+        };
+#pragma unroll
+        for (int i = 0; i < 2 * AL; i++) dma_a(0, i);
+#pragma unroll
+        for (int g = 0; g < NSW; g++) dma_w(g, 0, g);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm((NSW - 1) * 4, 15));
+        barrier();
+        /* Step s waits for the weights of the next step: issued 3 steps ago,
+         * before the loads of the last two. After the barrier it issues its
+         * patch loads, then the weights of step g + 4 (past the last step,
+         * the last chunk's again). A macro: the wait is an immediate. */
+#define CONV_STEP(s)                                                                                               \
+    do {                                                                                                           \
+        __builtin_amdgcn_s_waitcnt(                                                                                \
+            waitcnt_imm(8 + (((s) + 8) % 9 < AL ? 2 : 0) + (((s) + 7) % 9 < AL ? 2 : 0), 15));                     \
+        barrier();                                                                                                 \
+        if ((s) < AL) {                                                                                            \
+            dma_a(chunk + 1, (s) < AL ? 2 * (s) : 0);                                                              \
+            dma_a(chunk + 1, (s) < AL ? 2 * (s) + 1 : 0);                                                          \
+        }                                                                                                          \
+        dma_w(st, min(chunk + ((s) + NSW) / 9, chunks - 1), ((s) + NSW) % 9);                                      \
+        st = (st + 1) & (NSW - 1);                                                                                 \
+    } while (0)
+        for (int chunk = 0, st = 0; chunk < chunks; chunk++) {
+            CONV_STEP(0); CONV_STEP(1); CONV_STEP(2);
+            CONV_STEP(3); CONV_STEP(4); CONV_STEP(5);
+            CONV_STEP(6); CONV_STEP(7); CONV_STEP(8);
+        }
+#undef CONV_STEP
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));   /* no DMA outstanding past here */
+    }
+    const int wm = (wave >> 1) & 1, wn = wave & 1;
+    f32x4 acc[FM_][FN_];
+    if (wave < 4) {
+#pragma unroll
+    for (int i = 0; i < FM_; i++)
+#pragma unroll
+        for (int j = 0; j < FN_; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[i][j][r] = 0.0f;
+    /* lane addresses of the patch per tap column and half, of the weights per half */
+    int ab[3][2], wb[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++) {
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) {
+            const int c = UP ? ((lr + dx - 1) >> 1) + 1 : lr + dx;
+            ab[dx][kk] = (wm * (UP ? 4 : 8) * PW + c) * 128 + (((kk * 4 + lg) ^ ((c >> 1) & 7)) << 4);
+        }
+        wb[kk] = swz(wn * 64 + lr, kk * 4 + lg) * 2;
+    }
+    bf16x8 a0[FM_], w0[FN_], a1[FM_], w1[FN_];
+    auto frags = [&](int buf, int st, int s, int kk, bf16x8 (&a)[FM_], bf16x8 (&w)[FN_]) {
+        const char *const pa = sm + buf * A_BYTES + ab[s % 3][kk], *const pw = wring + st * W_BYTES + wb[kk];
+#pragma unroll
+        for (int ni = 0; ni < FN_; ni++) w[ni] = *(const bf16x8 *)(pw + ni * 16 * BK * 2);
+#pragma unroll
+        for (int mi = 0; mi < FM_; mi++) {
+            const int r = UP ? ((mi + s / 3 - 1) >> 1) + 1 : mi + s / 3;
+            a[mi] = *(const bf16x8 *)(pa + r * PW * 128);
+        }
+    };
+    auto mfmas = [&](const bf16x8 (&a)[FM_], const bf16x8 (&w)[FN_]) {
+#pragma unroll
+        for (int mi = 0; mi < FM_; mi++)
+#pragma unroll
+            for (int ni = 0; ni < FN_; ni++)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[ni], a[mi], acc[mi][ni], 0, 0, 0);
+    };
+    auto interleave = [&]() {
+#pragma unroll
+        for (int i = 0; i < FM_ + FN_; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        }
+    };
+    barrier();   /* chunk 0's patch, step 0's weights */
+    frags(0, 0, 0, 0, a0, w0);
+    for (int chunk = 0, st = 0; chunk < chunks; chunk++) {
+#pragma unroll
+        for (int s = 0; s < 9; s++) {
+            frags(chunk & 1, st, s, 1, a1, w1);
+            mfmas(a0, w0);
+            interleave();
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
+            barrier();
+            st = (st + 1) & (NSW - 1);
+            frags(s == 8 ? (chunk + 1) & 1 : chunk & 1, st, (s + 1) % 9, 0, a0, w0);
+            mfmas(a1, w1);
+            interleave();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    }
+
+    /* The tile leaves through LDS (free now), as f32 rows of 128 channels and
+     * 16 bytes: all eight waves store it, 32 lanes a whole pixel row, and the
+     * residual is in flight meanwhile. Thread t has the 4 channels 4 (t % 32)
+     * of pixels t / 32 + 16 i. Pixels outside the image take an address inside
+     * it and are not stored. */
+    constexpr int OSTR = 132;
+    static_assert(256 * OSTR * 4 <= 2 * A_BYTES + NSW * W_BYTES || UP, "the f32 tile fits the rings");
+    float *const ot = (float *)sm;
+    const int c4 = tid & 31, pr0 = tid >> 5, col = n0 + c4 * 4;
+    const bool part = P.ws != nullptr;   /* a split's partial sums: plain f32 rows of cout channels */
+    void *const out = part ? (void *)(P.ws + split * P.ws_stride) : P.out;
+    const int epi = part ? IRIS_EPI_F32 : P.epi, ldo = part ? P.cout : P.ldo;
+    const float *const bias = part ? nullptr : P.bias;
+    size_t off[16];
+    float4 res[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {   /* i: the tile's pixel row, pr0: its column */
+        off[i] = ((size_t)min(y0 + i, P.H - 1) * P.W + min(x0 + pr0, P.W - 1)) * ldo + col;
+        if (epi == IRIS_EPI_ADD) res[i] = *(const float4 *)((const float *)out + off[i]);
+    }
+    __syncthreads();   /* every read and every load of the rings is done */
+    if (wave < 4) {
+#pragma unroll
+        for (int mi = 0; mi < FM_; mi++)
+#pragma unroll
+            for (int ni = 0; ni < FN_; ni++)
+                *(f32x4 *)(ot + ((wm * 8 + mi) * 16 + lr) * OSTR + wn * 64 + ni * 16 + lg * 4) = acc[mi][ni];
+    }
+    __syncthreads();
+    const float4 v = bias ? *(const float4 *)(bias + col) : make_float4(0, 0, 0, 0);
+    float s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const bool on = y0 + i < P.H && x0 + pr0 < P.W;
+        const float4 q = *(const float4 *)(ot + (i * 16 + pr0) * OSTR + c4 * 4);
+        float4 r = make_float4(q.x + v.x, q.y + v.y, q.z + v.z, q.w + v.w);
+        if (epi == IRIS_EPI_ADD) {
+            r.x += res[i].x; r.y += res[i].y; r.z += res[i].z; r.w += res[i].w;
+        }
+        if (on) {
+            if (epi == IRIS_EPI_BF16)
+                *(uint2 *)((uint16_t *)out + off[i]) =
+                    make_uint2((uint32_t)f2bf_hw(r.x) | ((uint32_t)f2bf_hw(r.y) << 16),
+                               (uint32_t)f2bf_hw(r.z) | ((uint32_t)f2bf_hw(r.w) << 16));
+            else
+                *(float4 *)((float *)out + off[i]) = r;
+            s1 += (r.x + r.y) + (r.z + r.w);
+            s2 += (r.x * r.x + r.y * r.y) + (r.z * r.z + r.w * r.w);
+        }
+    }
+    if (gn) {
+        /* per thread the sums of 4 channels over 16 pixels, then the 16
+         * threads of the channels and the group's chunks in order, in f64 */
+        gnl[pr0][c4][0] = s1;
+        gnl[pr0][c4][1] = s2;
+        __syncthreads();
+        const int cpg = P.cout / P.gn_groups;
+        if (tid < 128 / cpg) {
+            double s = 0.0, q = 0.0;
+            for (int c = tid * cpg / 4; c < (tid + 1) * cpg / 4; c++)
+                for (int m = 0; m < 16; m++) {
+                    s += (double)gnl[m][c][0];
+                    q += (double)gnl[m][c][1];
+                }
+            double *dst = P.gn_part + ((size_t)tile * P.gn_groups + n0 / cpg + tid) * 2;
+            dst[0] = s;
+            dst[1] = q;
+        }
+    }
+}
+
+template <bool UP> int launch_patch(const ConvParams &P) {
+    constexpr int PW = UP ? 10 : 18;
+    /* the rings, or the f32 tile of the epilogue */
+    constexpr size_t ring = 2 * ((PW * PW + 7) / 8) * 1024 + 4 * 128 * BK * 2, ot = 256 * 132 * 4;
+    constexpr size_t smem = ring > ot ? ring : ot;
+    static std::once_flag once;
+    static hipError_t attr = hipSuccess;
+    std::call_once(once, [] {
+        attr = hipFuncSetAttribute((const void *)conv3x3_patch_kernel<UP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)smem);
+    });
+    if (iris_check(attr, "conv3x3 smem attribute")) return -1;
+    IRIS_LAUNCH((conv3x3_patch_kernel<UP>), dim3(8 * P.per_xcd), dim3(512), smem, iris_stream(), P);
+    return iris_launch_check("conv3x3_patch_kernel");
+}
+
+}  // namespace
+
+extern "C" int iris_hip_conv3x3_tiled(const iris_conv3x3_t *c, int *gn_blocks) {
+    if (gn_blocks) *gn_blocks = 0;
+    auto other = [&]() {
+        if (gn_blocks && c && c->gn_part) *gn_blocks = (c->H * c->W + 255) / 256;
+        return iris_hip_conv3x3(c);
+    };
+    if (!c || (c->up != 0 && c->up != 1) || c->H <= 0 || c->W <= 0 || c->cout <= 0 || c->splits > 1) return other();
+    const int cus = iris_cu_count();
+    const long long ty = (c->H + 15) / 16, tx = (c->W + 15) / 16, tiles = ty * tx * (c->cout / 128);
+    const double area = (double)c->H * c->W;
+    /* Tiles past one round may overshoot the image by a third (the products
+     * of the overshoot cost time there; at 1.13, 90 x 166, they still win);
+     * within a round they only use idle CUs. Few tiles are split over the
+     * input channels by an estimate (us): 0.5 per K step, 8 per block, the
+     * partials written and read at 2.2 TB/s with one launch more, and a
+     * statistics pass where the sums were asked for: 64 x 64 pixels, 512 ->
+     * 512 (64 tiles) 56 us + 9 us of reduce pass in the 256-row kernel, split
+     * by 2 or 4 here 35. */
+    if (c->cout % 128 || c->ldo % 4 || (((uintptr_t)c->out | (uintptr_t)c->bias) & 15) || tiles >= (1LL << 28) ||
+        (tiles > cus && 256.0 * ty * tx > 1.35 * area))
+        return other();
+    GemmParams chk;
+    if (conv_params(c, 128, chk)) return -1;
+    const int chunks = c->cin / BK;
+    const bool can = c->ws && !((uintptr_t)c->ws & 15);
+    int splits = 1;
+    double best = 1e30;
+    for (int s = 1; s <= 8 && s <= chunks; s *= 2) {
+        const double part = 4.0 * area * c->cout;
+        if (s > 1 && (!can || tiles * s > cus || s * part > (double)c->ws_bytes)) break;
+        const double us = 9.0 * ((chunks + s - 1) / s) * 0.5 + 8.0 +
+                          (s > 1 ? (s + 1) * part / 2.2e6 + 5.0 + (c->gn_part ? 7.0 : 0.0) : 0.0);
+        if (us < best) { best = us; splits = s; }
+    }
+    ConvParams P;
+    memset(&P, 0, sizeof(P));
+    P.in = c->in; P.wt = c->wt; P.out = c->out; P.bias = c->bias;
+    P.H = c->H; P.W = c->W; P.cin = c->cin; P.cout = c->cout; P.ldo = c->ldo; P.epi = c->epi;
+    P.tx = (int)tx; P.tn = c->cout / 128; P.tiles = (int)tiles;
+    P.cps = (chunks + splits - 1) / splits;
+    P.total = P.tiles * splits; P.per_xcd = (P.total + 7) / 8;
+    P.in_bytes = chk.conv_in_bytes;
+    if (splits == 1) {
+        P.gn_part = c->gn_part; P.gn_groups = c->gn_groups;
+        if (gn_blocks && c->gn_part) *gn_blocks = (int)(ty * tx);
+        return c->up ? launch_patch<true>(P) : launch_patch<false>(P);
+    }
+    P.ws = c->ws;
+    P.ws_stride = (long long)c->H * c->W * c->cout;
+    if (c->up ? launch_patch<true>(P) : launch_patch<false>(P)) return -1;
+    return launch_reduce(&chk.p[0], &P.ws, &P.ws_stride, &splits, 1);
 }

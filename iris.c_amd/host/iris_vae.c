@@ -532,25 +532,27 @@ static int conv(iris_vae_gpu_t *v, const uint16_t *in, const uint16_t *w, const 
     c.up = up;
     c.ldo = cout;
     c.epi = epi;
-    /* fewer tiles than CUs: split K (9 cin) over blocks */
-    const long long tiles = ((long long)H * W + 255) / 256 * ((cout + 255) / 256);
-    int splits = 1;
-    while (tiles * splits * 2 <= 256 && splits < 4 && 9 * cin / 64 / (splits * 2) >= 8) splits *= 2;
-    if (splits > 1 && (size_t)splits * H * W * cout * sizeof(float) <= v->ws_bytes) {
-        c.splits = splits;
-        c.ws = v->ws;
-        c.ws_bytes = v->ws_bytes;
+    stats = stats && cout % (4 * VAE_GROUPS) == 0;
+    c.ws = v->ws;
+    c.ws_bytes = v->ws_bytes;
+    if (up == 2 || cout % 128) {
+        /* fewer 256-row tiles than CUs: split K (9 cin) over blocks */
+        const long long tiles = ((long long)H * W + 255) / 256 * ((cout + 255) / 256);
+        int splits = 1;
+        while (tiles * splits * 2 <= 256 && splits < 4 && 9 * cin / 64 / (splits * 2) >= 8) splits *= 2;
+        if (splits > 1 && (size_t)splits * H * W * cout * sizeof(float) <= v->ws_bytes) c.splits = splits;
+        stats = stats && c.splits <= 1;
     }
-    stats = stats && c.splits <= 1 && cout % (4 * VAE_GROUPS) == 0;
     if (stats) {
         c.gn_part = v->part;
         c.gn_groups = VAE_GROUPS;
     }
     v->st_buf = NULL;
-    if (iris_hip_conv3x3(&c)) return -1;
-    if (stats) {
+    int nblk = 0;
+    if (iris_hip_conv3x3_tiled(&c, &nblk)) return -1;
+    if (nblk > 0) {
         v->st_buf = out;
-        v->st_nblk = (H * W + 255) / 256;
+        v->st_nblk = nblk;
     }
     return 0;
 }

@@ -1,0 +1,123 @@
+"""iris_hip_conv3x3_tiled: 3x3 convolutions on 16 x 16 pixel tiles, against
+float64, and the GroupNorm sums of each tile."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import iris_testlib as tl
+
+pytestmark = pytest.mark.gpu
+EPI_F32, EPI_BF16, EPI_ADD = 0, 1, 5
+
+
+@pytest.fixture(scope="module")
+def lib():
+    lib = tl.hip()
+    lib.iris_hip_conv3x3_tiled.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    return lib
+
+
+def bf(x):
+    return tl.bf16_to_f32(tl.to_bf16(x))
+
+
+def conv64(x, w, b, up):
+    if up:
+        x = x.repeat(2, 0).repeat(2, 1)
+    H, W = x.shape[:2]
+    xp = np.pad(x.astype(np.float64), ((1, 1), (1, 1), (0, 0)))
+    out = np.zeros((H, W, w.shape[0])) + b
+    for tap in range(9):
+        dy, dx = tap // 3, tap % 3
+        out += xp[dy:dy + H, dx:dx + W] @ w[:, tap].astype(np.float64).T
+    return out
+
+
+@pytest.mark.parametrize("H,W,cin,cout,up,tiled", [
+    (176, 192, 64, 128, 0, True),      # one channel chunk, whole tiles
+    (173, 190, 128, 128, 0, True),     # two chunks (both patch buffers), ragged on both sides
+    (96, 97, 256, 512, 0, True),       # four chunks, four channel tiles
+    (160, 208, 64, 256, 1, True),      # through the upsample
+    (150, 190, 128, 256, 1, True),     # upsample, ragged
+    (1, 1, 64, 128, 0, True),          # one pixel
+    (16, 17, 64, 128, 0, True),    # two tiles
+    (170, 193, 64, 192, 0, False),     # a part-empty channel tile: the other kernel
+])
+def test_conv3x3_tiled(lib, H, W, cin, cout, up, tiled):
+    """Every epilogue against float64 (f32 sums: 1e-5; bf16 output: 4e-3),
+    repeatable bit for bit, which kernel ran, and with the sums requested the
+    sum and sum of squares per tile and group of what was written."""
+    G = 32
+    rng = np.random.default_rng(H + W + cin)
+    x = bf(rng.standard_normal((H >> up, W >> up, cin)).astype(np.float32))
+    w = bf((rng.standard_normal((cout, 9, cin)) / np.sqrt(9 * cin)).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    ref = conv64(x, w, b, up)
+    dx, dw, db = tl.Dev.of(tl.to_bf16(x)), tl.Dev.of(tl.to_bf16(w)), tl.Dev.of(b)
+    x0 = rng.standard_normal((H, W, cout)).astype(np.float32)
+    ty, tx = -(-H // 16), -(-W // 16)
+    gn = cout % (4 * G) == 0
+    for epi in (EPI_F32, EPI_BF16, EPI_ADD):
+        got = []
+        for _ in range(2):
+            o = tl.Dev(H * W * cout * 2) if epi == EPI_BF16 else tl.Dev.of(x0)
+            part = tl.Dev.of(np.zeros((max(ty * tx, -(-H * W // 256)), G, 2)))
+            c = tl.Conv3x3(dx.ptr, dw.ptr, o.ptr, db.ptr, H, W, cin, cout, up, cout, epi, 1, None, 0,
+                           part.ptr if gn else None, G if gn else 0)
+            n = ctypes.c_int(-1)
+            assert lib.iris_hip_profile_enable(1) == 0
+            assert lib.iris_hip_conv3x3_tiled(ctypes.byref(c), ctypes.byref(n)) == 0, lib.iris_hip_last_error()
+            recs = (tl.KernelTime * 4)()
+            assert lib.iris_hip_profile_read(recs, 4) == 1 and lib.iris_hip_profile_enable(0) == 0
+            assert (b"patch" in recs[0].kernel) == tiled, recs[0].kernel
+            assert n.value == (0 if not gn else ty * tx if tiled else -(-H * W // 256))
+            got.append((o.get(np.uint16 if epi == EPI_BF16 else np.float32, (H, W, cout)),
+                        part.get(np.float64, (max(ty * tx, -(-H * W // 256)), G, 2))))
+            o.close()
+        assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+        y = tl.bf16_to_f32(got[0][0]) if epi == EPI_BF16 else got[0][0]
+        want = ref + x0 if epi == EPI_ADD else ref
+        assert tl.rel_l2(y, want) < (4e-3 if epi == EPI_BF16 else 1e-5)
+        if gn and tiled:
+            pad = np.zeros((ty * 16, tx * 16, cout))
+            pad[:H, :W] = want
+            t = pad.reshape(ty, 16, tx, 16, G, cout // G)
+            sums = np.stack([t.sum((1, 3, 5)), (t * t).sum((1, 3, 5))], -1).reshape(ty * tx, G, 2)
+            # f32 sums of 256 x 4 .. 16 values: their rounding against the sum of magnitudes
+            np.testing.assert_allclose(got[0][1], sums, rtol=1e-4, atol=2e-2)
+
+
+@pytest.mark.parametrize("H,W,cin,cout,up", [(32, 32, 512, 512, 0), (20, 22, 256, 128, 1), (16, 16, 512, 256, 0),
+                                             (33, 18, 512, 128, 0)])
+def test_conv3x3_tiled_split(lib, H, W, cin, cout, up):
+    """Few tiles and a workspace: split over the input channels, partials
+    reduced in order: every epilogue against float64, repeatable; no sums."""
+    rng = np.random.default_rng(H + cin)
+    x = bf(rng.standard_normal((H >> up, W >> up, cin)).astype(np.float32))
+    w = bf((rng.standard_normal((cout, 9, cin)) / np.sqrt(9 * cin)).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    ref = conv64(x, w, b, up)
+    dx, dw, db = tl.Dev.of(tl.to_bf16(x)), tl.Dev.of(tl.to_bf16(w)), tl.Dev.of(b)
+    x0 = rng.standard_normal((H, W, cout)).astype(np.float32)
+    nb = 8 * H * W * cout * 4
+    ws, part = tl.Dev(nb), tl.Dev(4096 * 64 * 8)
+    for epi in (EPI_F32, EPI_BF16, EPI_ADD):
+        got, split = [], False
+        for _ in range(2):
+            o = tl.Dev(H * W * cout * 2) if epi == EPI_BF16 else tl.Dev.of(x0)
+            c = tl.Conv3x3(dx.ptr, dw.ptr, o.ptr, db.ptr, H, W, cin, cout, up, cout, epi, 0, ws.ptr, nb, part.ptr, 32)
+            n = ctypes.c_int(-1)
+            assert lib.iris_hip_profile_enable(1) == 0
+            assert lib.iris_hip_conv3x3_tiled(ctypes.byref(c), ctypes.byref(n)) == 0, lib.iris_hip_last_error()
+            recs = (tl.KernelTime * 4)()
+            k = lib.iris_hip_profile_read(recs, 4)
+            assert lib.iris_hip_profile_enable(0) == 0
+            names = [r.kernel for r in recs[:k]]
+            split = any(b"reduce" in m for m in names)
+            assert any(b"patch" in m for m in names) and (n.value == 0) == split, (names, n.value)
+            got.append(o.get(np.uint16 if epi == EPI_BF16 else np.float32, (H, W, cout)))
+            o.close()
+        assert split and np.array_equal(got[0], got[1])
+        y = tl.bf16_to_f32(got[0]) if epi == EPI_BF16 else got[0]
+        assert tl.rel_l2(y, ref + x0 if epi == EPI_ADD else ref) < (4e-3 if epi == EPI_BF16 else 1e-5)
