@@ -281,6 +281,23 @@ typedef struct {
 } iris_norm_args_t;
 int iris_hip_rownorm(const iris_norm_args_t *a);
 
+/* No counterpart in the reference. iris_hip_gemm_fill_n, then the row passes
+ * that follow it: with x set (one problem, F32 epilogue without a vec) Z-Image's
+ * gated residual of its output, iris_hip_rms_gated_add(x, out, w, gate, M, N,
+ * eps, 0); with norm set iris_hip_rownorm(norm). The same bits as the calls one
+ * after the other. Where the products are split over K and norm reads their
+ * rows in order (GATED_ADD into norm->x, or x == norm->x), one launch sums the
+ * partials, updates the rows and normalises them; the output of a product with
+ * x set is then not written. */
+typedef struct {
+    float *x;
+    const float *w, *gate;
+    float eps;
+    const iris_norm_args_t *norm;
+} iris_row_tail_t;
+int iris_hip_gemm_fill_tail(const iris_gemm_problem_t *problems, int n_problems, float *d_workspace,
+                            size_t workspace_bytes, const iris_row_tail_t *tail);
+
 /* Z-Image gated residual: x[r,:] += g[:] * RMSNorm(y[r,:]) * w[:] with
  * g = gate (gate_tanh 0), tanh(gate) (gate_tanh 1), or 1 when gate is NULL. */
 int iris_hip_rms_gated_add(float *d_x, const float *d_y, const float *d_w, const float *d_gate,

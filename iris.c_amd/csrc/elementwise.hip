@@ -22,24 +22,12 @@ namespace {
 
 constexpr int NT = 256;
 
-/* One block of 256 threads per row: thread t owns float4 columns t, t + 256,
- * ... (V of them); each reduction is a wave shuffle plus a 4-entry LDS sum.
- * A wave per row leaves each wave a long chain (load, two reductions, store)
- * over 12 KB; spreading the row over four waves shortens it and keeps more
- * rows' loads in flight (5.5 TB/s against 4.8 for wave-per-row at
- * 4608 x 3072 f32 -> bf16). */
+/* The normalisation of one row held in v (column chunk t + i NT): rownorm's
+ * arithmetic, shared with the kernels that update the row first. */
 template <int V, int MODE>
-__global__ __launch_bounds__(NT) void rownorm_kernel(const iris_norm_args_t a) {
-    __shared__ float red[2][NT / IRIS_WAVE];
-    const int row = blockIdx.x, t = threadIdx.x, wv = t >> 6, lane = t & 63;
-    const float *x = a.x + (size_t)row * a.ldx;
-    const int nv = a.cols >> 2;
-    float4 v[V];
-#pragma unroll
-    for (int i = 0; i < V; i++) {
-        const int c = t + i * NT;
-        v[i] = c < nv ? ld_stream((const float4 *)x + c) : make_float4(0, 0, 0, 0);
-    }
+__device__ __forceinline__ void norm_row(const iris_norm_args_t &a, int row, const float4 (&v)[V],
+                                         float (&red)[2][NT / IRIS_WAVE]) {
+    const int t = threadIdx.x, wv = t >> 6, lane = t & 63, nv = a.cols >> 2;
     const bool use_b = (a.period ? row % a.period : row) >= a.split;
     const float *shift = use_b ? a.shiftB : a.shiftA;
     const float *scale = use_b ? a.scaleB : a.scaleA;
@@ -108,6 +96,96 @@ __global__ __launch_bounds__(NT) void rownorm_kernel(const iris_norm_args_t a) {
             *(float4 *)((float *)a.out + (size_t)row * a.ldo + 4 * c) = make_float4(y[0], y[1], y[2], y[3]);
         }
     }
+}
+
+/* One block of 256 threads per row: thread t owns float4 columns t, t + 256,
+ * ... (V of them); each reduction is a wave shuffle plus a 4-entry LDS sum.
+ * A wave per row leaves each wave a long chain (load, two reductions, store)
+ * over 12 KB; spreading the row over four waves shortens it and keeps more
+ * rows' loads in flight (5.5 TB/s against 4.8 for wave-per-row at
+ * 4608 x 3072 f32 -> bf16). */
+template <int V, int MODE>
+__global__ __launch_bounds__(NT) void rownorm_kernel(const iris_norm_args_t a) {
+    __shared__ float red[2][NT / IRIS_WAVE];
+    const int row = blockIdx.x, t = threadIdx.x, nv = a.cols >> 2;
+    const float *x = a.x + (size_t)row * a.ldx;
+    float4 v[V];
+#pragma unroll
+    for (int i = 0; i < V; i++) {
+        const int c = t + i * NT;
+        v[i] = c < nv ? ld_stream((const float4 *)x + c) : make_float4(0, 0, 0, 0);
+    }
+    norm_row<V, MODE>(a, row, v, red);
+}
+
+/* What follows a product split over K, in one launch of a block per row: the
+ * chunks' partials summed in chunk order, the residual update of the row
+ * (x += vec * s, or with SAND Z-Image's x += g * RMSNorm(s) * w), and the
+ * normalisation of the updated row for the next product (MODE, or NORM_NONE).
+ * Bits as splitk_reduce_kernel, rms_gated_add_kernel and rownorm_kernel one
+ * after the other, without writing and reading the row between them and two
+ * launches less. Same box, whole passes, us: Z-Image at 512 x 512 (1120 rows)
+ * 2139 -> 2050, Flux at 256 x 256 (768 rows) 1419 -> 1385 and 512 x 512 2072 ->
+ * 2045, the text encode of 512 rows 6541 -> 6397. */
+constexpr int NORM_NONE = 3;
+template <int V, int MODE, bool SAND>
+__global__ __launch_bounds__(NT) void reduce_rows_kernel(const iris_reduce_rows_t R) {
+    __shared__ float red[2][NT / IRIS_WAVE], rs[NT / IRIS_WAVE];
+    const int row = blockIdx.x, t = threadIdx.x, nv = R.cols >> 2;
+    int pi = 0;
+#pragma unroll
+    for (int i = 1; i < 4; i++)
+        if (i < R.n && row >= R.start[i]) pi = i;
+    const float *ws = R.ws[pi] + (size_t)(row - R.start[pi]) * R.cols;
+    float *const xr = R.x + (size_t)row * R.ldx;
+    const float *const vec = R.vec[pi];
+    const long long stride = R.stride[pi];
+    const int splits = R.chunks[pi];
+    float4 v[V], xo[V];
+#pragma unroll
+    for (int i = 0; i < V; i++) {
+        const int c = t + i * NT;
+        v[i] = make_float4(0, 0, 0, 0);
+        xo[i] = c < nv ? ((const float4 *)xr)[c] : make_float4(0, 0, 0, 0);
+    }
+#pragma unroll 4
+    for (int k = 0; k < splits; k++)
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+            const int c = t + i * NT;
+            if (c >= nv) continue;
+            const float4 q = ld_stream((const float4 *)(ws + k * stride) + c);
+            v[i].x += q.x; v[i].y += q.y; v[i].z += q.z; v[i].w += q.w;
+        }
+    float inv = 0.0f;
+    if constexpr (SAND) {
+        float q = 0.0f;
+#pragma unroll
+        for (int i = 0; i < V; i++) q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+        q = wave_sum(q);
+        if ((t & 63) == 0) rs[t >> 6] = q;
+        __syncthreads();
+        inv = 1.0f / sqrtf(((rs[0] + rs[1]) + (rs[2] + rs[3])) / R.cols + R.eps);
+    }
+#pragma unroll
+    for (int i = 0; i < V; i++) {
+        const int c = t + i * NT;
+        if (c >= nv) continue;
+        float4 g4 = make_float4(1, 1, 1, 1);
+        if (vec) g4 = ((const float4 *)vec)[c];
+        if constexpr (SAND) {
+            const float4 w4 = ((const float4 *)R.w)[c];
+            const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w}, ww[4] = {w4.x, w4.y, w4.z, w4.w};
+            const float gg[4] = {g4.x, g4.y, g4.z, g4.w};
+            float *xp = &xo[i].x;
+#pragma unroll
+            for (int j = 0; j < 4; j++) xp[j] += gg[j] * (e[j] * inv * ww[j]);
+        } else {
+            xo[i].x += g4.x * v[i].x; xo[i].y += g4.y * v[i].y; xo[i].z += g4.z * v[i].z; xo[i].w += g4.w * v[i].w;
+        }
+        ((float4 *)xr)[c] = xo[i];
+    }
+    if constexpr (MODE != NORM_NONE) norm_row<V, MODE>(R.norm, row, xo, red);
 }
 
 /* x += g * RMSNorm(y) * w, one block of 256 threads per row (as rownorm). */
@@ -471,9 +549,10 @@ int grid1d(size_t n) {
 
 extern "C" {
 
-int iris_hip_rownorm(const iris_norm_args_t *a) {
-    if (a->rows <= 0) return 0;
-    /* float4 columns per thread of a 256-thread block */
+/* checks a normalisation; b: its arguments with a weight set that no row
+ * selects (it may be left NULL) standing in for the other; *v: float4 columns
+ * per thread of a 256-thread block */
+static int norm_args(const iris_norm_args_t *a, iris_norm_args_t &b, int *pv) {
     const int need = (a->cols / 4 + NT - 1) / NT;
     static const int vs[] = {1, 2, 3, 4, 6, 8, 12, 16};
     int v = 0;
@@ -482,8 +561,7 @@ int iris_hip_rownorm(const iris_norm_args_t *a) {
     if (a->cols % 4 || a->cols <= 0 || !v) return iris_set_error("rownorm: cols=%d", a->cols);
     if (a->ldx % 4 || a->ldo % 4) return iris_set_error("rownorm: ld must be multiple of 4");
     if (a->mode < IRIS_NORM_LN_MOD || a->mode > IRIS_NORM_RMS) return iris_set_error("rownorm: mode %d", a->mode);
-    /* a set that no row selects may be left NULL: it stands in for the other */
-    iris_norm_args_t b = *a;
+    b = *a;
     const bool only_a = !b.period && b.split >= b.rows, only_b = !b.period && b.split <= 0;
     if (only_a) { b.shiftB = b.shiftA; b.scaleB = b.scaleA; b.wB = b.wA; }
     if (only_b) { b.shiftA = b.shiftB; b.scaleA = b.scaleB; b.wA = b.wB; }
@@ -491,6 +569,15 @@ int iris_hip_rownorm(const iris_norm_args_t *a) {
         return iris_set_error("rownorm: LN_MOD needs scale and shift for the row sets in use");
     if (b.mode == IRIS_NORM_RMS && (!b.wA || !b.wB)) return iris_set_error("rownorm: RMS needs weights");
     if (b.mode == IRIS_NORM_LN_SCALE && (!b.scaleA || !b.scaleB)) return iris_set_error("rownorm: LN_SCALE needs scales");
+    *pv = v;
+    return 0;
+}
+
+int iris_hip_rownorm(const iris_norm_args_t *a) {
+    if (a->rows <= 0) return 0;
+    iris_norm_args_t b;
+    int v;
+    if (norm_args(a, b, &v)) return -1;
     const dim3 grid(a->rows);
 #define ROWNORM_CASE(VV)                                                                                          \
     case VV:                                                                                                      \
@@ -508,6 +595,37 @@ int iris_hip_rownorm(const iris_norm_args_t *a) {
 #undef ROWNORM_CASE
     return iris_launch_check("rownorm_kernel");
 }
+
+}  /* extern "C" */
+
+int iris_reduce_rows(const iris_reduce_rows_t *r, int rows) {
+    iris_reduce_rows_t R = *r;
+    int v = (R.cols / 4 + NT - 1) / NT, mode = NORM_NONE;
+    if (R.has_norm) {
+        if (norm_args(&r->norm, R.norm, &v)) return -1;
+        mode = R.norm.mode;
+    }
+    const bool sand = R.w != nullptr;
+    if (v < 1 || v > 4 || mode == IRIS_NORM_LN_SCALE || (!sand && mode == NORM_NONE))
+        return iris_set_error("reduce_rows: cols=%d mode=%d", R.cols, mode);
+    const dim3 grid(rows);
+#define ROWS_CASE(VV)                                                                                              \
+    case VV:                                                                                                       \
+        if (!sand && mode == IRIS_NORM_LN_MOD)                                                                     \
+            IRIS_LAUNCH((reduce_rows_kernel<VV, IRIS_NORM_LN_MOD, false>), grid, dim3(NT), 0, iris_stream(), R);   \
+        else if (!sand)                                                                                            \
+            IRIS_LAUNCH((reduce_rows_kernel<VV, IRIS_NORM_RMS, false>), grid, dim3(NT), 0, iris_stream(), R);      \
+        else if (mode == IRIS_NORM_RMS)                                                                            \
+            IRIS_LAUNCH((reduce_rows_kernel<VV, IRIS_NORM_RMS, true>), grid, dim3(NT), 0, iris_stream(), R);       \
+        else                                                                                                       \
+            IRIS_LAUNCH((reduce_rows_kernel<VV, NORM_NONE, true>), grid, dim3(NT), 0, iris_stream(), R);           \
+        break;
+    switch (v) { ROWS_CASE(1) ROWS_CASE(2) ROWS_CASE(3) ROWS_CASE(4) }
+#undef ROWS_CASE
+    return iris_launch_check("reduce_rows_kernel");
+}
+
+extern "C" {
 
 int iris_hip_rms_gated_add(float *x, const float *y, const float *w, const float *gate, int rows, int cols,
                            float eps, int gate_tanh) {

@@ -1181,6 +1181,70 @@ int check_problem(const iris_gemm_problem_t &p) {
 
 namespace {
 
+/* the row passes of iris_hip_gemm_fill_tail; done: the reduce launch took them */
+struct RowTail {
+    const iris_row_tail_t *t;
+    bool done;
+};
+
+/* whether one row pass over the partials of these split problems (nr of n in
+ * the launch) is what t asks for: whole rows of at most 4096 columns in 16-byte
+ * chunks, in the order of the rows it updates */
+bool tail_fits(const iris_gemm_problem_t *ps, float *const *ws, int nr, int n, const iris_row_tail_t &t) {
+    const bool sand = t.x != nullptr;
+    if (nr != n || (sand && n != 1) || (!sand && !t.norm)) return false;
+    const int N = ps[0].N;
+    const float *const x = sand ? t.x : t.norm->x;
+    const int ldx = sand ? N : t.norm->ldx;
+    long long rows = 0;
+    for (int i = 0; i < n; i++) {
+        const iris_gemm_problem_t &p = ps[i];
+        if (p.N != N || ((uintptr_t)ws[i] & 15) || ((uintptr_t)p.vec & 15)) return false;
+        if (sand ? p.epi != IRIS_EPI_F32 || p.vec : p.epi != IRIS_EPI_GATED_ADD || p.ldo != ldx ||
+                                                         (const float *)p.out != x + rows * ldx)
+            return false;
+        rows += p.M;
+    }
+    /* a block per row: fewer rows than half the CUs leave the sums of many
+     * chunks to too few of them (37 rows: text encode 2802 us with the separate
+     * passes, 2934 in one) */
+    if (rows * 2 < iris_cu_count()) return false;
+    if (N % 4 || N > 4096 || ldx % 4 || ldx < N || ((uintptr_t)x & 15)) return false;
+    if (sand && (((uintptr_t)t.w | (uintptr_t)t.gate) & 15)) return false;
+    if (!t.norm) return true;
+    const iris_norm_args_t &a = *t.norm;
+    return a.x == x && a.ldx == ldx && a.cols == N && a.rows == rows &&
+           (sand ? a.mode == IRIS_NORM_RMS : a.mode == IRIS_NORM_RMS || a.mode == IRIS_NORM_LN_MOD);
+}
+
+int launch_tail(const iris_gemm_problem_t *ps, float *const *ws, const long long *stride, const int *chunks, int n,
+                const iris_row_tail_t &t) {
+    iris_reduce_rows_t R;
+    memset(&R, 0, sizeof(R));
+    int rows = 0;
+    for (int i = 0; i < n; i++) {
+        R.ws[i] = ws[i];
+        R.vec[i] = t.x ? t.gate : ps[i].vec;
+        R.stride[i] = stride[i];
+        R.chunks[i] = chunks[i];
+        R.start[i] = rows;
+        rows += ps[i].M;
+    }
+    R.n = n;
+    R.cols = ps[0].N;
+    R.x = t.x ? t.x : (float *)ps[0].out;
+    R.ldx = t.x ? ps[0].N : ps[0].ldo;
+    if (t.x) {
+        R.w = t.w;
+        R.eps = t.eps;
+    }
+    if (t.norm) {
+        R.has_norm = 1;
+        R.norm = *t.norm;
+    }
+    return iris_reduce_rows(&R, rows);
+}
+
 /* One launch of up to MAXP problems. want[i] > 1 (want may be NULL) splits
  * problem i over K into that many chunks of whole K steps: its f32 partials
  * go to the workspace (after those of the split problems before it) and one
@@ -1194,7 +1258,7 @@ namespace {
  * round); bnt > 0 forces the tile width. bmt = 128: 128 x 256 tiles (no
  * second K segment). */
 int launch_gemm(const iris_gemm_problem_t *probs, int n, const int *want, float *ws, size_t ws_bytes,
-                int phase1 = 0, int force_bnt = 0, int bmt = BM, int ring = RING_NONE) {
+                int phase1 = 0, int force_bnt = 0, int bmt = BM, int ring = RING_NONE, RowTail *tail = nullptr) {
     if (!probs || n < 1 || n > MAXP) return iris_set_error("gemm: %d problems (1..%d)", n, MAXP);
     if (ring) bmt = RING_BM[ring];
     GemmParams P;
@@ -1287,6 +1351,10 @@ int launch_gemm(const iris_gemm_problem_t *probs, int n, const int *want, float 
             rstride[nr] = P.ws_stride[i];
             rchunks[nr++] = P.chunks[i];
         }
+    if (tail && tail_fits(rp, rws, nr, n, *tail->t)) {
+        tail->done = true;
+        return launch_tail(rp, rws, rstride, rchunks, nr, *tail->t);
+    }
     return launch_reduce(rp, rws, rstride, rchunks, nr);
 }
 
@@ -1489,7 +1557,9 @@ RingPlan ring_plan(const iris_gemm_problem_t *probs, int n, int cus, size_t ws_b
 
 }  // namespace
 
-extern "C" int iris_hip_gemm_fill_n(const iris_gemm_problem_t *probs, int n, float *ws, size_t ws_bytes) {
+namespace {
+
+int fill_impl(const iris_gemm_problem_t *probs, int n, float *ws, size_t ws_bytes, RowTail *tail) {
     if (!probs || n < 1 || n > MAXP) return iris_set_error("gemm_fill: %d problems (1..%d)", n, MAXP);
     const int cus = iris_cu_count();
     long long tiles = 0, tiles128 = 0;
@@ -1536,15 +1606,15 @@ extern "C" int iris_hip_gemm_fill_n(const iris_gemm_problem_t *probs, int n, flo
         const RingPlan r = ring_plan(probs, n, cus, ws_bytes);
         if (r.ring && r.us < 0.97 * std::min(est(false, s256), s128 > 0 ? est(true, s128) : 1e30)) {
             for (int i = 0; i < n; i++) want[i] = r.splits;
-            return launch_gemm(probs, n, r.splits > 1 ? want : nullptr, ws, ws_bytes, 0, 0, BM, r.ring);
+            return launch_gemm(probs, n, r.splits > 1 ? want : nullptr, ws, ws_bytes, 0, 0, BM, r.ring, tail);
         }
         if (s128 > 0 && est(true, s128) < est(false, s256)) {
             for (int i = 0; i < n; i++) want[i] = s128;
-            return launch_gemm(probs, n, s128 > 1 ? want : nullptr, ws, ws_bytes, 0, 0, 128);
+            return launch_gemm(probs, n, s128 > 1 ? want : nullptr, ws, ws_bytes, 0, 0, 128, RING_NONE, tail);
         }
         if (s256 > 1) {
             for (int i = 0; i < n; i++) want[i] = s256;
-            return launch_gemm(probs, n, want, ws, ws_bytes);
+            return launch_gemm(probs, n, want, ws, ws_bytes, 0, 0, BM, RING_NONE, tail);
         }
     }
     if (n == 1 && ws && !((uintptr_t)ws & 15)) {
@@ -1557,6 +1627,26 @@ extern "C" int iris_hip_gemm_fill_n(const iris_gemm_problem_t *probs, int n, flo
         }
     }
     return launch_gemm(probs, n, nullptr, nullptr, 0);
+}
+
+}  // namespace
+
+extern "C" int iris_hip_gemm_fill_n(const iris_gemm_problem_t *probs, int n, float *ws, size_t ws_bytes) {
+    return fill_impl(probs, n, ws, ws_bytes, nullptr);
+}
+
+extern "C" int iris_hip_gemm_fill_tail(const iris_gemm_problem_t *probs, int n, float *ws, size_t ws_bytes,
+                                       const iris_row_tail_t *tail) {
+    if (!probs || !tail || (tail->x && (n != 1 || probs->epi != IRIS_EPI_F32 || probs->vec || probs->ldo != probs->N ||
+                                        !tail->w)))
+        return iris_set_error("gemm_fill_tail: a gated residual follows one F32 product of contiguous rows");
+    RowTail t = {tail, false};
+    if (fill_impl(probs, n, ws, ws_bytes, &t)) return -1;
+    if (t.done) return 0;
+    if (tail->x && iris_hip_rms_gated_add(tail->x, (const float *)probs->out, tail->w, tail->gate, probs->M, probs->N,
+                                          tail->eps, 0))
+        return -1;
+    return tail->norm ? iris_hip_rownorm(tail->norm) : 0;
 }
 
 extern "C" int iris_hip_gemm_ring(const iris_gemm_problem_t *probs, int n, int rows, int splits, float *ws,

@@ -9,6 +9,22 @@ int iris_set_error(const char *fmt, ...);
 int iris_check(hipError_t e, const char *what);
 int iris_launch_check(const char *what);
 
+/* Row pass after products split over K (iris_hip_gemm_fill_tail): the
+ * partials of up to 4 problems (rows start[i] .. of problem i, chunks[i] of
+ * them stride[i] apart) update the rows of x, then norm is taken of them. vec:
+ * the gate per column (NULL: 1); w: Z-Image's RMSNorm of the product's row
+ * with this weight and eps before the gate (NULL: none). */
+typedef struct {
+    const float *ws[4], *vec[4];
+    long long stride[4];
+    int chunks[4], start[4], n, cols, ldx, has_norm;
+    float *x;
+    const float *w;
+    float eps;
+    iris_norm_args_t norm;
+} iris_reduce_rows_t;
+int iris_reduce_rows(const iris_reduce_rows_t *r, int rows);
+
 /* Per-launch timing for the library's profile (iris_hip_profile_enable):
  * while enabled and the stream is not being captured, each launch is
  * bracketed by two events on the library stream. begin returns the record

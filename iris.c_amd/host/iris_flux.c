@@ -753,8 +753,8 @@ static int attention(iris_transformer_t *tf, const float *wqA, const float *wqB,
     return iris_hip_attention(&a);
 }
 
-static int adaln(iris_transformer_t *tf, const float *shA, const float *scA, const float *shB, const float *scB,
-                 int split) {
+static iris_norm_args_t adaln(iris_transformer_t *tf, const float *shA, const float *scA, const float *shB,
+                              const float *scB, int split) {
     work_t *w = &tf->w;
     iris_norm_args_t a;
     memset(&a, 0, sizeof(a));
@@ -762,12 +762,32 @@ static int adaln(iris_transformer_t *tf, const float *shA, const float *scA, con
     a.rows = w->B * w->S; a.cols = tf->hidden; a.mode = IRIS_NORM_LN_MOD; a.eps = 1e-6f;
     a.split = split; a.period = w->S;
     a.shiftA = shA; a.scaleA = scA; a.shiftB = shB; a.scaleB = scB;
-    return iris_hip_rownorm(&a);
+    return a;
+}
+
+/* the first normalisation of a block: every double block's, every single block's */
+enum { NEXT_NONE, NEXT_DOUBLE, NEXT_SINGLE };
+static iris_norm_args_t first_norm(iris_transformer_t *tf, int kind) {
+    const int h = tf->hidden;
+    const float *mi = tf->w.mod, *mt = mi + 6 * h, *ms = mi + 12 * h;
+    return kind == NEXT_DOUBLE ? adaln(tf, mt, mt + h, mi, mi + h, tf->w.T) : adaln(tf, ms, ms + h, ms, ms + h, tf->w.S);
+}
+
+/* residual products, then the normalisation of the updated rows that reads
+ * them next (NULL: none), in one row pass where the products are split over K */
+static int gemm_norm(iris_transformer_t *tf, const iris_gemm_problem_t *p, int n, const iris_norm_args_t *norm) {
+    if (!norm) return gemm_fill(tf, p, n);
+    iris_row_tail_t t;
+    memset(&t, 0, sizeof(t));
+    t.norm = norm;
+    return iris_hip_gemm_fill_tail(p, n, tf->w.fill_ws, FILL_WS_BYTES, &t);
 }
 
 /* double_block_forward, iris_transformer_flux.c:2366-2614: per batch slot,
- * txt rows [0, T) use the txt weights/modulation, img rows [T, S) the img ones. */
-static int double_block_forward(iris_transformer_t *tf, int i) {
+ * txt rows [0, T) use the txt weights/modulation, img rows [T, S) the img ones.
+ * normed: the block before left this one's normalised rows in a; next: the
+ * block whose this one leaves. */
+static int double_block_forward(iris_transformer_t *tf, int i, int normed, int next) {
     work_t *w = &tf->w;
     const dev_double_t *bw = &tf->dbl[i];
     int h = tf->hidden, mlp = tf->mlp, T = w->T, I = w->I, S = w->S, B = w->B, hm = h + mlp;
@@ -777,7 +797,8 @@ static int double_block_forward(iris_transformer_t *tf, int i) {
     const lora_dev_t *l_iq = lora_at(tf, 4 * i), *l_ip = lora_at(tf, 4 * i + 1);
     const lora_dev_t *l_tq = lora_at(tf, 4 * i + 2), *l_tp = lora_at(tf, 4 * i + 3);
     /* AdaLN (shift1, scale1) -> Q, K, V per stream */
-    CK(adaln(tf, mt, mt + h, mi, mi + h, T));
+    iris_norm_args_t nrm = first_norm(tf, NEXT_DOUBLE);
+    if (!normed) CK(iris_hip_rownorm(&nrm));
     n = 0;
     for (int b = 0; b < B; b++) {
         size_t r0 = (size_t)b * S;
@@ -805,9 +826,9 @@ static int double_block_forward(iris_transformer_t *tf, int i) {
                     IRIS_EPI_GATED_ADD);
         lora_seg(tf, &p[n++], l_ip, r0 + T, 0);
     }
-    CK(gemm_fill(tf, p, n));
     /* AdaLN (shift2, scale2) -> SwiGLU FFN -> gated residual (gate2) */
-    CK(adaln(tf, mt + 3 * h, mt + 4 * h, mi + 3 * h, mi + 4 * h, T));
+    nrm = adaln(tf, mt + 3 * h, mt + 4 * h, mi + 3 * h, mi + 4 * h, T);
+    CK(gemm_norm(tf, p, n, &nrm));
     n = 0;
     for (int b = 0; b < B; b++) {
         size_t r0 = (size_t)b * S;
@@ -824,18 +845,20 @@ static int double_block_forward(iris_transformer_t *tf, int i) {
         p[n++] = prob(w->cat + (r0 + T) * hm + h, hm, bw->img_down, mlp, w->x + (r0 + T) * h, h, mi + 5 * h, I, h, mlp,
                       IRIS_EPI_GATED_ADD);
     }
-    CK(gemm_fill(tf, p, n));
+    if (next) nrm = first_norm(tf, next);
+    CK(gemm_norm(tf, p, n, next ? &nrm : NULL));
     return 0;
 }
 
-/* single_block_forward, iris_transformer_flux.c:3761-3928 */
-static int single_block_forward(iris_transformer_t *tf, int i) {
+/* single_block_forward, iris_transformer_flux.c:3761-3928; normed, next as double_block_forward */
+static int single_block_forward(iris_transformer_t *tf, int i, int normed, int next) {
     work_t *w = &tf->w;
     const dev_single_t *bw = &tf->sgl[i];
     int h = tf->hidden, mlp = tf->mlp, hm = h + mlp, BS = w->B * w->S;
     const float *ms = w->mod + 12 * h;                   /* shift scale gate */
     const lora_dev_t *l1 = lora_at(tf, 4 * tf->n_double + 2 * i), *l2 = lora_at(tf, 4 * tf->n_double + 2 * i + 1);
-    CK(adaln(tf, ms, ms + h, ms, ms + h, w->S));
+    iris_norm_args_t nrm = first_norm(tf, NEXT_SINGLE);
+    if (!normed) CK(iris_hip_rownorm(&nrm));
     /* the first linear's two parts: Q,K,V rows -> qkv; gate/up rows -> SwiGLU
      * -> cat[:, h:] */
     iris_gemm_problem_t p[2];
@@ -868,7 +891,8 @@ static int single_block_forward(iris_transformer_t *tf, int i) {
     CK(lora_down(tf, l2, w->cat, hm, 0, BS));
     p[0] = prob(w->cat, hm, bw->out, hm, w->x, h, ms + 2 * h, BS, h, hm, IRIS_EPI_GATED_ADD);
     lora_seg(tf, &p[0], l2, 0, 0);
-    CK(gemm_fill(tf, p, 1));
+    if (next) nrm = first_norm(tf, next);
+    CK(gemm_norm(tf, p, 1, next ? &nrm : NULL));
     return 0;
 }
 
@@ -919,8 +943,10 @@ static int enqueue_forward(iris_transformer_t *tf) {
     /* once forked, the side stream is joined whatever failed after the fork */
     if (side && iris_hip_join() && !rc) rc = -1;
     CK(rc);
-    for (int i = 0; i < tf->n_double; i++) CK(double_block_forward(tf, i));
-    for (int i = 0; i < tf->n_single; i++) CK(single_block_forward(tf, i));
+    const int nd = tf->n_double, ns = tf->n_single;
+    for (int i = 0; i < nd; i++)
+        CK(double_block_forward(tf, i, i > 0, i + 1 < nd ? NEXT_DOUBLE : ns > 0 ? NEXT_SINGLE : NEXT_NONE));
+    for (int i = 0; i < ns; i++) CK(single_block_forward(tf, i, nd + i > 0, i + 1 < ns ? NEXT_SINGLE : NEXT_NONE));
     /* final layer on the target rows: AdaLN with (scale, shift) order, proj_out,
      * written transposed to NCHW (:4254-4301) */
     const float *fm = w->mod + 15 * h;
@@ -945,14 +971,14 @@ static int enqueue_forward(iris_transformer_t *tf) {
 int iris_flux_double_block_forward(iris_transformer_t *tf, int idx) {
     if (!tf->w.valid || idx < 0 || idx >= tf->n_double) return -1;
     if (lora_sync(tf) < 0 || lora_work(tf) < 0) return -1;
-    if (double_block_forward(tf, idx)) return -1;
+    if (double_block_forward(tf, idx, 0, NEXT_NONE)) return -1;
     return iris_hip_sync();
 }
 
 int iris_flux_single_block_forward(iris_transformer_t *tf, int idx) {
     if (!tf->w.valid || idx < 0 || idx >= tf->n_single) return -1;
     if (lora_sync(tf) < 0 || lora_work(tf) < 0) return -1;
-    if (single_block_forward(tf, idx)) return -1;
+    if (single_block_forward(tf, idx, 0, NEXT_NONE)) return -1;
     return iris_hip_sync();
 }
 

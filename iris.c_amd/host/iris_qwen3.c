@@ -389,21 +389,32 @@ static int gemm(qwen3_model_t *m, const iris_gemm_problem_t *p) {
     return iris_hip_gemm_fill(p, m->ws, m->ws_bytes);
 }
 
-static int rms(const qwen3_model_t *m, const float *w, int S) {
+static iris_norm_args_t rms(const qwen3_model_t *m, const float *w, int S) {
     iris_norm_args_t a;
     memset(&a, 0, sizeof(a));
     a.x = m->x; a.ldx = m->hidden; a.out = m->a; a.ldo = m->hidden; a.out_bf16 = 1;
     a.rows = S; a.cols = m->hidden; a.mode = IRIS_NORM_RMS; a.eps = QWEN3_RMS_NORM_EPS;
     a.split = S; a.wA = w; a.wB = w;
-    return iris_hip_rownorm(&a);
+    return a;
 }
 
-/* qwen3_layer_forward (iris_qwen3.c:496-538) */
-static int layer_forward(qwen3_model_t *m, const qlayer_t *l, int S, int n_real) {
+/* a residual product, then the RMSNorm of the updated rows that reads them
+ * next (w NULL: none), in one row pass where the product is split over K */
+static int gemm_rms(qwen3_model_t *m, const iris_gemm_problem_t *p, const float *w, int S) {
+    if (!w) return gemm(m, p);
+    const iris_norm_args_t a = rms(m, w, S);
+    iris_row_tail_t t;
+    memset(&t, 0, sizeof(t));
+    t.norm = &a;
+    return iris_hip_gemm_fill_tail(p, 1, m->ws, m->ws_bytes, &t);
+}
+
+/* qwen3_layer_forward (iris_qwen3.c:496-538), from its normalised input rows
+ * to those of the next layer (next_ln1 NULL: the last one) */
+static int layer_forward(qwen3_model_t *m, const qlayer_t *l, const float *next_ln1, int S, int n_real) {
     const int h = m->hidden, qd = m->heads * HD, kd = m->kv_heads * HD, I = m->inter;
     const int S_pad = (S + 63) / 64 * 64;
     iris_gemm_problem_t p;
-    CK(rms(m, l->ln1, S));
     p = prob(m->a, h, l->qkv, h, m->qkv, qd + 2 * kd, S, qd + 2 * kd, h, IRIS_EPI_BF16);
     CK(gemm(m, &p));
     iris_qkprep_args_t q;
@@ -428,12 +439,11 @@ static int layer_forward(qwen3_model_t *m, const qlayer_t *l, int S, int n_real)
     CK(iris_hip_attention(&at));
     /* o_proj + residual (:461-466, :514-517) */
     p = prob(m->attn, qd, l->o, qd, m->x, h, S, h, qd, IRIS_EPI_GATED_ADD);
-    CK(gemm(m, &p));
-    CK(rms(m, l->ln2, S));
+    CK(gemm_rms(m, &p, l->ln2, S));
     p = prob(m->a, h, l->gate_up, h, m->mlp, I, S, 2 * I, h, IRIS_EPI_SWIGLU);
     CK(gemm(m, &p));
     p = prob(m->mlp, I, l->down, I, m->x, h, S, h, I, IRIS_EPI_GATED_ADD);
-    CK(gemm(m, &p));
+    CK(gemm_rms(m, &p, next_ln1, S));
     return 0;
 }
 
@@ -468,8 +478,13 @@ float *qwen3_forward(qwen3_model_t *m, const int *input_ids, const int *attentio
         fail("embedding");
         return NULL;
     }
+    const iris_norm_args_t first = rms(m, m->L[0].ln1, S);
+    if (iris_hip_rownorm(&first)) {
+        fail("input norm");
+        return NULL;
+    }
     for (int i = 0; i <= last; i++) {
-        if (layer_forward(m, &m->L[i], S, n_real)) return NULL;
+        if (layer_forward(m, &m->L[i], i < last ? m->L[i + 1].ln1 : NULL, S, n_real)) return NULL;
         int slot = -1;
         if (m->mode) slot = i == last ? 0 : -1;
         else slot = i == QWEN3_OUTPUT_LAYER_1 ? 0 : i == QWEN3_OUTPUT_LAYER_2 ? 1 : i == QWEN3_OUTPUT_LAYER_3 ? 2 : -1;

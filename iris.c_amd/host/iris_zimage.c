@@ -469,27 +469,44 @@ static int zgemm(zi_transformer_t *tf, const iris_gemm_problem_t *p) {
     return iris_hip_gemm_fill(p, tf->w.fill_ws, ZI_FILL_WS_BYTES);
 }
 
-static int rms(zi_transformer_t *tf, const float *x, uint16_t *out, int rows, const float *w, const float *scale) {
+static iris_norm_args_t rms(zi_transformer_t *tf, const float *x, uint16_t *out, int rows, const float *w,
+                            const float *scale) {
     iris_norm_args_t a;
     memset(&a, 0, sizeof(a));
     a.x = x; a.ldx = tf->dim; a.out = out; a.ldo = tf->dim; a.out_bf16 = 1;
     a.rows = rows; a.cols = tf->dim; a.mode = IRIS_NORM_RMS; a.eps = ZI_EPS;
     a.split = rows; a.wA = w; a.scaleA = scale;
-    return iris_hip_rownorm(&a);
+    return a;
+}
+
+/* a product into y, x += gate * RMSNorm(y) * w, and the normalisation of the
+ * updated rows that reads them next (norm NULL: none); one row pass over the
+ * partials where the product is split over K */
+static int zgemm_add(zi_transformer_t *tf, const iris_gemm_problem_t *p, float *x, const float *w, const float *gate,
+                     const iris_norm_args_t *norm) {
+    iris_row_tail_t t;
+    memset(&t, 0, sizeof(t));
+    t.x = x; t.w = w; t.gate = gate; t.eps = ZI_EPS; t.norm = norm;
+    return iris_hip_gemm_fill_tail(p, 1, tf->w.fill_ws, ZI_FILL_WS_BYTES, &t);
 }
 
 /* zi_block_forward (:790-870) on rows [r0, r0 + n) of the unified sequence;
  * keys outside [klo0, khi0) U [klo1, khi1) (relative to r0) are padding. mod
  * is NULL for the unmodulated context refiner, else 1+scale_msa | gate_msa |
  * 1+scale_mlp | gate_mlp, the gates already through tanh (iris_hip_tanh_cols
- * after the modulation GEMV). */
+ * after the modulation GEMV). normed: the rows' first normalisation is in a
+ * already (the block before left it); next, next_mod: the block that reads the
+ * same rows after this one, whose first normalisation this one ends with, or
+ * NULL. */
 static int zi_block_forward(zi_transformer_t *tf, const zi_dev_block_t *b, const float *mod, int r0, int n,
-                            int klo0, int khi0, int klo1, int khi1) {
+                            int klo0, int khi0, int klo1, int khi1, int normed, const zi_dev_block_t *next,
+                            const float *next_mod) {
     zi_work_t *w = &tf->w;
     int d = tf->dim, f = tf->ffn;
     float *x = w->x + (size_t)r0 * d;
     /* attention: h = attention(norm1(x) * (1 + scale_msa)) */
-    CK(rms(tf, x, w->a, n, b->n1, mod));
+    iris_norm_args_t nrm = rms(tf, x, w->a, n, b->n1, mod);
+    if (!normed) CK(iris_hip_rownorm(&nrm));
     iris_gemm_problem_t p = zprob(w->a, d, b->qkv, w->qkv, 3 * d, NULL, n, 3 * d, d, IRIS_EPI_BF16);
     CK(zgemm(tf, &p));
     iris_qkprep_args_t q;
@@ -513,17 +530,16 @@ static int zi_block_forward(zi_transformer_t *tf, const zi_dev_block_t *b, const
     at.rope_cos = w->rp_cos + (size_t)r0 * 64; at.rope_sin = w->rp_sin + (size_t)r0 * 64;
     at.ws = w->attn_ws; at.ws_bytes = w->attn_ws_bytes;
     CK(iris_hip_attention(&at));
+    /* x += tanh(gate_msa) * norm2(attn_out), then the FFN's input:
+     * x += tanh(gate_mlp) * norm2(w2(silu(w1 h) * w3 h)), h = norm1(x) * (1 + scale_mlp) */
     p = zprob(w->attn, d, b->o, w->y, d, NULL, n, d, d, IRIS_EPI_F32);
-    CK(zgemm(tf, &p));
-    /* x += tanh(gate_msa) * norm2(attn_out) */
-    CK(iris_hip_rms_gated_add(x, w->y, b->n2, mod ? mod + d : NULL, n, d, ZI_EPS, 0));
-    /* FFN: x += tanh(gate_mlp) * norm2(w2(silu(w1 h) * w3 h)), h = norm1(x) * (1 + scale_mlp) */
-    CK(rms(tf, x, w->a, n, b->fn1, mod ? mod + 2 * d : NULL));
+    nrm = rms(tf, x, w->a, n, b->fn1, mod ? mod + 2 * d : NULL);
+    CK(zgemm_add(tf, &p, x, b->n2, mod ? mod + d : NULL, &nrm));
     p = zprob(w->a, d, b->w13, w->ffn, f, NULL, n, 2 * f, d, IRIS_EPI_SWIGLU);
     CK(zgemm(tf, &p));
     p = zprob(w->ffn, f, b->w2, w->y, d, NULL, n, d, f, IRIS_EPI_F32);
-    CK(zgemm(tf, &p));
-    CK(iris_hip_rms_gated_add(x, w->y, b->fn2, mod ? mod + 3 * d : NULL, n, d, ZI_EPS, 0));
+    if (next) nrm = rms(tf, x, w->a, n, next->n1, next_mod);
+    CK(zgemm_add(tf, &p, x, b->fn2, mod ? mod + 3 * d : NULL, next ? &nrm : NULL));
     return 0;
 }
 
@@ -559,14 +575,19 @@ static int zi_enqueue(zi_transformer_t *tf) {
     CK(zgemm(tf, &p));
     CK(iris_hip_fill_rows(w->x, tf->cap_pad, Ip + w->cap_len, U, d));
     /* refiners: noise refiner on image rows, context refiner on caption rows */
-    for (int i = 0; i < tf->refiners; i++)
-        CK(zi_block_forward(tf, &tf->nr[i], w->mods + (size_t)i * 4 * d, 0, Ip, 0, I, 0, 0));
-    for (int i = 0; i < tf->refiners; i++)
-        CK(zi_block_forward(tf, &tf->cr[i], NULL, Ip, Cp, 0, w->cap_len, 0, 0));
+    const int R = tf->refiners, L = tf->layers;
+#define MOD(k) (w->mods + (size_t)(k) * 4 * d)
+    for (int i = 0; i < R; i++)
+        CK(zi_block_forward(tf, &tf->nr[i], MOD(i), 0, Ip, 0, I, 0, 0, i > 0, i + 1 < R ? &tf->nr[i + 1] : NULL,
+                            MOD(i + 1)));
+    for (int i = 0; i < R; i++)
+        CK(zi_block_forward(tf, &tf->cr[i], NULL, Ip, Cp, 0, w->cap_len, 0, 0, i > 0,
+                            i + 1 < R ? &tf->cr[i + 1] : NULL, NULL));
     /* main layers on the unified [image | caption] sequence */
-    for (int i = 0; i < tf->layers; i++)
-        CK(zi_block_forward(tf, &tf->ly[i], w->mods + (size_t)(tf->refiners + i) * 4 * d, 0, U, 0, I, Ip,
-                            Ip + w->cap_len));
+    for (int i = 0; i < L; i++)
+        CK(zi_block_forward(tf, &tf->ly[i], MOD(R + i), 0, U, 0, I, Ip, Ip + w->cap_len, i > 0,
+                            i + 1 < L ? &tf->ly[i + 1] : NULL, MOD(R + i + 1)));
+#undef MOD
     /* final layer on the image rows: LayerNorm (eps 1e-6) * scale, linear + b, unpatchify */
     memset(&a, 0, sizeof(a));
     a.x = w->x; a.ldx = d; a.out = w->a; a.ldo = d; a.out_bf16 = 1;
@@ -586,15 +607,15 @@ int zi_block_forward_resident(zi_transformer_t *tf, int kind, int idx) {
     const int d = tf->dim;
     if (!w->valid || kind < 0 || kind > 2 || idx < 0 || idx >= (kind == 2 ? tf->layers : tf->refiners)) return -1;
     if (kind == 1) {
-        if (zi_block_forward(tf, &tf->cr[idx], NULL, w->Ip, w->Cp, 0, w->cap_len, 0, 0)) return -1;
+        if (zi_block_forward(tf, &tf->cr[idx], NULL, w->Ip, w->Cp, 0, w->cap_len, 0, 0, 0, NULL, NULL)) return -1;
         return iris_hip_sync();
     }
     const zi_dev_block_t *b = kind == 0 ? &tf->nr[idx] : &tf->ly[idx];
     float *mod = w->mods + (size_t)(kind == 0 ? idx : tf->refiners + idx) * 4 * d;
     if (iris_hip_gemv(mod, b->ada_w, w->temb, b->ada_b, 4 * d, tf->adaln_dim, 0)) return -1;
     if (iris_hip_tanh_cols(mod, 2, 2 * d, d, d)) return -1;
-    if (kind == 0 ? zi_block_forward(tf, b, mod, 0, w->Ip, 0, w->I, 0, 0)
-                  : zi_block_forward(tf, b, mod, 0, w->U, 0, w->I, w->Ip, w->Ip + w->cap_len))
+    if (kind == 0 ? zi_block_forward(tf, b, mod, 0, w->Ip, 0, w->I, 0, 0, 0, NULL, NULL)
+                  : zi_block_forward(tf, b, mod, 0, w->U, 0, w->I, w->Ip, w->Ip + w->cap_len, 0, NULL, NULL))
         return -1;
     return iris_hip_sync();
 }
