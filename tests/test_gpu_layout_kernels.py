@@ -36,6 +36,14 @@ def test_f32_to_bf16(lib, n, skip):
     assert np.array_equal(got[~nan], want[~nan]) and np.all(np.isnan(tl.bf16_to_f32(got[nan])))
 
 
+@pytest.mark.parametrize("C,hw", [(128, 1), (128, 31), (128, 33), (128, 256), (96, 65), (40, 32)])
+def test_nchw_to_tokens(lib, C, hw):
+    x = np.random.default_rng(hw).standard_normal((C, hw)).astype(np.float32)
+    d, o = tl.Dev.of(x), tl.Dev(C * hw * 2)
+    assert lib.iris_hip_nchw_to_tokens(o.ptr, d.ptr, C, hw) == 0
+    assert np.array_equal(o.get(np.uint16, (hw, C)), tl.to_bf16(np.ascontiguousarray(x.T)))
+
+
 @pytest.mark.parametrize("N,K,act", [(8192, 3072, 1), (8195, 520, 0), (17 * 512, 512, 1), (8192, 4096, 0)])
 def test_gemv_rows(lib, N, K, act):
     """Products of enough rows for four to a wave, a ragged last wave: the
