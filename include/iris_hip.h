@@ -35,6 +35,15 @@ void *iris_hip_malloc(size_t bytes);                 /* NULL on failure */
 void iris_hip_free(void *d_ptr);
 int iris_hip_memcpy_h2d(void *d_dst, const void *src, size_t bytes);   /* on the stream */
 int iris_hip_memcpy_d2h(void *dst, const void *d_src, size_t bytes);   /* synchronous */
+/* Download beside later work of the library stream: pinned memory of the
+ * caller's, and a copy into it on the side stream, ordered after everything
+ * enqueued on the library stream so far; iris_hip_download_wait returns when
+ * the copy of that slot (0..7) is done. d_src is not rewritten before that.
+ * Not for captured work. */
+void *iris_hip_host_malloc(size_t bytes);            /* NULL on failure */
+void iris_hip_host_free(void *ptr);
+int iris_hip_download(void *pinned_dst, const void *d_src, size_t bytes, int slot);
+int iris_hip_download_wait(int slot);
 int iris_hip_memcpy_d2d(void *d_dst, const void *d_src, size_t bytes); /* on the stream */
 int iris_hip_memset(void *d_dst, int value, size_t bytes);             /* not for captured work */
 int iris_hip_sync(void);

@@ -208,6 +208,40 @@ int iris_hip_memcpy_d2h(void *dst, const void *src, size_t bytes) {
     return iris_check(hipStreamSynchronize(g_stream), "sync after d2h");
 }
 
+void *iris_hip_host_malloc(size_t bytes) {
+    void *p = nullptr;
+    if (!iris_hip_available()) return nullptr;
+    if (hipHostMalloc(&p, bytes ? bytes : 256, hipHostMallocDefault) != hipSuccess) {
+        iris_set_error("hipHostMalloc(%zu) failed", bytes);
+        return nullptr;
+    }
+    return p;
+}
+
+void iris_hip_host_free(void *p) {
+    if (p) (void)hipHostFree(p);
+}
+
+/* events behind the copies of iris_hip_download, made on first use */
+static hipEvent_t g_down_ev[8], g_down_at;
+
+int iris_hip_download(void *dst, const void *src, size_t bytes, int slot) {
+    if (slot < 0 || slot >= 8 || !iris_hip_available()) return iris_set_error("download slot %d", slot);
+    if (!g_down_at && iris_check(hipEventCreateWithFlags(&g_down_at, hipEventDisableTiming), "download event")) return -1;
+    if (!g_down_ev[slot] &&
+        iris_check(hipEventCreateWithFlags(&g_down_ev[slot], hipEventDisableTiming), "download event"))
+        return -1;
+    return iris_check(hipEventRecord(g_down_at, g_stream), "download order") ||
+           iris_check(hipStreamWaitEvent(g_side, g_down_at, 0), "download order") ||
+           iris_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g_side), "download") ||
+           iris_check(hipEventRecord(g_down_ev[slot], g_side), "download event");
+}
+
+int iris_hip_download_wait(int slot) {
+    if (slot < 0 || slot >= 8 || !g_down_ev[slot]) return iris_set_error("download slot %d", slot);
+    return iris_check(hipEventSynchronize(g_down_ev[slot]), "download wait");
+}
+
 int iris_hip_memcpy_d2d(void *dst, const void *src, size_t bytes) {
     if (!bytes) return 0;
     return iris_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, g_stream), "memcpy d2d");
