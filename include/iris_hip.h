@@ -266,6 +266,9 @@ int iris_hip_transpose_bf16(uint16_t *d_dst, int ld_dst, int rows_pad, const uin
  * f32 (or NULL) receives the conv output as [3][H][W]. */
 int iris_hip_vae_conv_out(uint8_t *d_rgb, float *d_f32, const uint16_t *d_g, int H, int W, int cin,
                           const float *d_wt, const float *d_bias);
+/* the same of swish(x * ab[c] + ab[cin + c]) with x f32 (gn_finalize's ab), kept in f32 */
+int iris_hip_vae_conv_out_norm(uint8_t *d_rgb, float *d_f32, const float *d_x, const float *d_ab, int H, int W,
+                               int cin, const float *d_wt, const float *d_bias);
 
 /* y[n] = act_out( sum_k W[n][k] * act_in(x[k]) + bias[n] ), W bf16 [N][K], x f32.
  * act_in: 0 none, 1 SiLU (expf). Used for the timestep MLP and modulation. */

@@ -14,14 +14,17 @@
  *   - denormalize + unpatchify + post_quant_conv (iris_vae.c:860-897): one
  *     kernel from the NCHW latent to the conv_in input;
  *   - the mid-block attention's softmax and V transpose (iris_vae.c:260-357);
- *   - conv_out 128 -> 3 and the [-1,1] -> uint8 conversion
- *     (iris_vae.c:968-994): one direct kernel.
+ *   - conv_out 128 -> 3 with its GroupNorm and swish and the [-1,1] -> uint8
+ *     conversion (iris_vae.c:968-994): one kernel on f32 MFMA.
  */
 #include "iris_internal.h"
+
+#include <mutex>
 
 namespace {
 
 constexpr int NT = 256;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void load8(const float *p, float v[8]) {
     const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 4);
@@ -324,106 +327,159 @@ __global__ __launch_bounds__(NT) void transpose_bf16_kernel(const uint16_t *src,
     }
 }
 
-/* conv_out (3x3, cin -> 3, zero padding) and the image conversion, one thread
- * per pixel: v = conv + bias; u8 = (uint8)(clamp(((v + 1) * 0.5) * 255, 0,
- * 255) + 0.5) in the reference's order of operations; f32 (if not NULL)
- * receives v as [3][H][W]. Weights wt[tap][cin][4] (4th lane zero) sit in
- * LDS and are read as one broadcast float4 per input channel. */
-__global__ __launch_bounds__(NT) void conv_out_kernel(const uint16_t *g, int H, int W, int cin, const float *wt,
-                                                      const float *bias, uint8_t *rgb, float *f32) {
-    extern __shared__ float4 wl[];
-    for (int i = threadIdx.x; i < 9 * cin; i += NT) wl[i] = ((const float4 *)wt)[i];
-    __syncthreads();
-    const int p = blockIdx.x * NT + threadIdx.x;
-    if (p >= H * W) return;
-    const int y = p / W, x = p % W;
-    float a0 = bias[0], a1 = bias[1], a2 = bias[2];
-    for (int tap = 0; tap < 9; tap++) {
-        const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-        if ((unsigned)yy >= (unsigned)H || (unsigned)xx >= (unsigned)W) continue;
-        const uint16_t *src = g + ((size_t)yy * W + xx) * cin;
-        const float4 *wr = wl + tap * cin;
-        for (int c = 0; c < cin; c += 8) {
-            float v[8];
-            load8(src + c, v);
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float4 k = wr[c + j];
-                a0 += v[j] * k.x;
-                a1 += v[j] * k.y;
-                a2 += v[j] * k.z;
-            }
-        }
-    }
-    const float o[3] = {a0, a1, a2};
-#pragma unroll
-    for (int ch = 0; ch < 3; ch++) {
-        if (f32) f32[(size_t)ch * H * W + p] = o[ch];
-        float val = (o[ch] + 1.0f) * 0.5f;
-        val = val * 255.0f;
-        if (val < 0) val = 0;
-        if (val > 255) val = 255;
-        rgb[(size_t)p * 3 + ch] = (uint8_t)(val + 0.5f);
-    }
-}
+/* conv_out (3x3, cin -> 3, zero padding) and the image conversion:
+ * v = conv + bias; u8 = (uint8)(clamp(((v + 1) * 0.5) * 255, 0, 255) + 0.5) in
+ * the reference's order of operations; f32 (if not NULL) receives v as
+ * [3][H][W]. A pixel's 27 products over its channels (9 taps x 3 outputs) are
+ * one row of a matrix product, formed once where the pixel is read, and an
+ * output sums the nine of its neighbours' rows: f32 MFMA (the weights are
+ * f32), K = cin, the 27 columns in two 16-row tiles. A block takes 30 x 16
+ * outputs: with their halo 32 x 18 pixels, 36 groups of 16 for 4 waves, whose
+ * rows of 27 (odd: consecutive pixels in different banks) fit in LDS beside
+ * the weights twice per CU. A lane holds 8 consecutive channels of its pixel
+ * per 32-channel step, the next 128 channels loading while the products of
+ * this 128 run. NORM: x is f32 and swish(x * ab[c] + ab[cin + c]) is taken on
+ * the way in, without a bf16 pass through memory. Blocks take tiles in order
+ * within an XCD's band, so a halo's second reading finds its L2.
+ * Bound by its products (64 f32 MFMAs per 16 pixels, halo 1.2 times) with the
+ * activation beside them: 1024 x 1024 x 128 in 187 us from f32, which replaces
+ * an apply pass of 196-212 and a kernel of one thread per output over
+ * LDS-staged tiles of 356; from bf16 about 180. */
+constexpr int CO_X = 30, CO_Y = 16, CO_W = CO_X + 2, CO_P = CO_W * (CO_Y + 2), CO_N = 27, CO_KC = 128;
+constexpr int CO_GW = CO_P / 16 / (NT / IRIS_WAVE);   /* groups of 16 pixels per wave */
+static_assert(CO_GW * 16 * (NT / IRIS_WAVE) == CO_P, "whole groups for every wave");
 
-/* The same convolution over 16 x 16 output tiles: the tile's input pixels
- * and their one-pixel halo are staged in LDS 32 channels at a time (each
- * input row read once per tile instead of once per tap and neighbour), the
- * chunk's weights beside them; one thread per output pixel. The sums run
- * chunk by chunk, tap by tap within a chunk. Rows of 32 channels are padded
- * to 40 elements, so the 16 pixels of a half wave read 16 distinct 4-bank
- * groups. */
-constexpr int CO_T = 16, CO_H = CO_T + 2, CO_C = 32, CO_STR = CO_C + 8;
-__global__ __launch_bounds__(NT) void conv_out_tiled_kernel(const uint16_t *g, int H, int W, int cin, const float *wt,
-                                                            const float *bias, uint8_t *rgb, float *f32) {
-    __shared__ __attribute__((aligned(16))) uint16_t xs[CO_H * CO_H * CO_STR];
-    __shared__ float4 wl[9 * CO_C];
-    const int tx = threadIdx.x & (CO_T - 1), ty = threadIdx.x / CO_T;
-    const int x0 = blockIdx.x * CO_T, y0 = blockIdx.y * CO_T;
-    float a0 = bias[0], a1 = bias[1], a2 = bias[2];
-    for (int c0 = 0; c0 < cin; c0 += CO_C) {
-        __syncthreads();   /* the previous chunk's reads are done */
-        for (int i = threadIdx.x; i < CO_H * CO_H * (CO_C / 8); i += NT) {
-            const int pix = i >> 2, part = i & 3;
-            const int gy = y0 + pix / CO_H - 1, gx = x0 + pix % CO_H - 1;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if ((unsigned)gy < (unsigned)H && (unsigned)gx < (unsigned)W)
-                v = *(const uint4 *)(g + ((size_t)gy * W + gx) * cin + c0 + part * 8);
-            *(uint4 *)(xs + pix * CO_STR + part * 8) = v;
-        }
-        for (int i = threadIdx.x; i < 9 * CO_C; i += NT) wl[i] = ((const float4 *)wt)[(i / CO_C) * cin + c0 + i % CO_C];
-        __syncthreads();
-        for (int tap = 0; tap < 9; tap++) {
-            const uint16_t *src = xs + ((ty + tap / 3) * CO_H + tx + tap % 3) * CO_STR;
-            const float4 *wr = wl + tap * CO_C;
+template <typename T, bool NORM>
+__global__ __launch_bounds__(NT, 2) void conv_out_kernel(const T *x, const float *ab, int H, int W, int cin,
+                                                         const float *wt, const float *bias, uint8_t *rgb, float *f32,
+                                                         int tx, int tiles, int per_xcd) {
+    extern __shared__ __attribute__((aligned(16))) float cosm[];
+    const int nch = (cin + CO_KC - 1) / CO_KC, tid = threadIdx.x, lane = tid & 63, q = lane >> 4, n = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float *rows = cosm, *wl = cosm + CO_P * CO_N, *abl = wl + nch * 32 * CO_KC;
+    /* wl[step][tile][half][lane][4]: channels 32 step + 8 (lane / 16) + 4 half.., column 16 tile + lane % 16
+     * (columns past the 27th stay unset: their rows of the product are not stored) */
+#pragma unroll 5
+    for (int i = tid; i < 9 * nch * CO_KC; i += NT) {
+        const int tap = i / (nch * CO_KC), c = i % (nch * CO_KC);
+        const float4 w4 = ((const float4 *)wt)[(size_t)tap * cin + (c < cin ? c : 0)];
+        const float w[3] = {w4.x, w4.y, w4.z};
 #pragma unroll
-            for (int c = 0; c < CO_C; c += 8) {
-                const u16x8 r = *(const u16x8 *)(src + c);
+        for (int o = 0; o < 3; o++) {
+            const int col = 3 * tap + o, ln = ((c >> 3) & 3) * 16 + (col & 15);
+            wl[((c >> 5) << 10) + ((col >> 4) << 9) + (((c >> 2) & 1) << 8) + ln * 4 + (c & 3)] = c < cin ? w[o] : 0.0f;
+        }
+    }
+    if (NORM)
+        for (int i = tid; i < 2 * nch * CO_KC; i += NT) {
+            const int c = i % (nch * CO_KC);
+            abl[i] = c < cin ? ab[i < nch * CO_KC ? c : cin + c] : 0.0f;
+        }
+    const int items = CO_GW * nch;
+    for (int k = blockIdx.x >> 3; k < per_xcd; k += gridDim.x >> 3) {
+        const int L = (blockIdx.x & 7) * per_xcd + k;
+        if (L >= tiles) break;
+        const int x0 = L % tx * CO_X, y0 = L / tx * CO_Y;
+        float raw[32];
+        auto inside = [&](int it) {
+            const int g = wave * CO_GW + it / nch, gy = y0 + (g >> 1) - 1, gx = x0 + (g & 1) * 16 + n - 1;
+            return (unsigned)gy < (unsigned)H && (unsigned)gx < (unsigned)W ? gy * W + gx : -1;
+        };
+        auto load = [&](int it) {
+            const int p = inside(it), c0 = it % nch * CO_KC + q * 8;
+            const T *src = x + (size_t)(p < 0 ? 0 : p) * cin;
+#pragma unroll
+            for (int s = 0; s < 4; s++) load8(src + (c0 + 32 * s < cin ? c0 + 32 * s : 0), raw + 8 * s);
+        };
+        load(0);
+        __syncthreads();   /* wl and abl are there; the last tile's rows are read */
+        f32x4 acc[2];
+#pragma unroll 1
+        for (int it = 0; it < items; it++) {
+            const int ch = it % nch, c0 = ch * CO_KC + q * 8;
+            const bool in = inside(it) >= 0;
+            float v[32];
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const uint32_t keep = in && c0 + 32 * s < cin ? ~0u : 0u;
+                float a[8], b[8];
+                if (NORM) {
+                    load8(abl + c0 + 32 * s, a);
+                    load8(abl + nch * CO_KC + c0 + 32 * s, b);
+                }
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
-                    const float v = bf2f(r[j]);
-                    const float4 k = wr[c + j];
-                    a0 += v * k.x;
-                    a1 += v * k.y;
-                    a2 += v * k.z;
+                    const float t = raw[8 * s + j];
+                    v[8 * s + j] = __uint_as_float(__float_as_uint(NORM ? silu_fast(t * a[j] + b[j]) : t) & keep);
+                }
+            }
+            if (it + 1 < items) load(it + 1);
+            if (ch == 0) acc[0] = acc[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const float *w = wl + ((ch * 4 + s) << 10) + lane * 4;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const f32x4 w0 = *(const f32x4 *)(w + 256 * h), w1 = *(const f32x4 *)(w + 512 + 256 * h);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[e], v[8 * s + 4 * h + e], acc[0], 0, 0, 0);
+                        acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[e], v[8 * s + 4 * h + e], acc[1], 0, 0, 0);
+                    }
+                }
+            }
+            if (ch == nch - 1) {
+                float *o = rows + ((wave * CO_GW + it / nch) * 16 + n) * CO_N + 4 * q;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    o[r] = acc[0][r];
+                    if (16 + 4 * q + r < CO_N) o[16 + r] = acc[1][r];
                 }
             }
         }
-    }
-    const int y = y0 + ty, x = x0 + tx;
-    if (y >= H || x >= W) return;
-    const int p = y * W + x;
-    const float o[3] = {a0, a1, a2};
+        __syncthreads();
+        for (int i = tid; i < CO_X * CO_Y; i += NT) {
+            const int px = i % CO_X, py = i / CO_X, xx = x0 + px, yy = y0 + py;
+            if (xx >= W || yy >= H) continue;
+            float o[3] = {bias[0], bias[1], bias[2]};
 #pragma unroll
-    for (int ch = 0; ch < 3; ch++) {
-        if (f32) f32[(size_t)ch * H * W + p] = o[ch];
-        float val = (o[ch] + 1.0f) * 0.5f;
-        val = val * 255.0f;
-        if (val < 0) val = 0;
-        if (val > 255) val = 255;
-        rgb[(size_t)p * 3 + ch] = (uint8_t)(val + 0.5f);
+            for (int tap = 0; tap < 9; tap++) {
+                const float *r = rows + ((py + tap / 3) * CO_W + px + tap % 3) * CO_N + 3 * tap;
+                o[0] += r[0];
+                o[1] += r[1];
+                o[2] += r[2];
+            }
+            const int p = yy * W + xx;
+#pragma unroll
+            for (int ch = 0; ch < 3; ch++) {
+                if (f32) f32[(size_t)ch * H * W + p] = o[ch];
+                float val = (o[ch] + 1.0f) * 0.5f;
+                val = val * 255.0f;
+                if (val < 0) val = 0;
+                if (val > 255) val = 255;
+                rgb[(size_t)p * 3 + ch] = (uint8_t)(val + 0.5f);
+            }
+        }
     }
+}
+
+template <typename T, bool NORM>
+int launch_conv_out(const T *x, const float *ab, int H, int W, int cin, const float *wt, const float *bias,
+                    uint8_t *rgb, float *f32) {
+    const int tx = (W + CO_X - 1) / CO_X, tiles = tx * ((H + CO_Y - 1) / CO_Y), per_xcd = (tiles + 7) / 8;
+    const int nch = (cin + CO_KC - 1) / CO_KC, round = (2 * iris_cu_count() + 7) / 8;
+    constexpr size_t most = sizeof(float) * (CO_P * CO_N + 2 * CO_KC * (32 + 2));   /* cin <= 256 */
+    const size_t smem = sizeof(float) * (CO_P * CO_N + nch * CO_KC * (32 + 2));
+    static std::once_flag once;
+    static hipError_t attr = hipSuccess;
+    std::call_once(once, [] {
+        attr = hipFuncSetAttribute((const void *)conv_out_kernel<T, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)most);
+    });
+    if (iris_check(attr, "conv_out smem attribute")) return -1;
+    IRIS_LAUNCH((conv_out_kernel<T, NORM>), dim3(8 * (per_xcd < round ? per_xcd : round)), dim3(NT), smem,
+                iris_stream(), x, ab, H, W, cin, wt, bias, rgb, f32, tx, tiles, per_xcd);
+    return iris_launch_check("conv_out_kernel");
 }
 
 unsigned blocks_for(size_t n) {
@@ -505,21 +561,21 @@ extern "C" int iris_hip_transpose_bf16(uint16_t *dst, int ld_dst, int rows_pad, 
     return iris_launch_check("transpose_bf16_kernel");
 }
 
+static bool conv_out_ok(const uint8_t *rgb, const void *x, int H, int W, int cin, const float *wt, const float *bias) {
+    return rgb && x && wt && bias && H > 0 && W > 0 && H <= 32768 && W <= 32768 && cin > 0 && cin <= 256 &&
+           cin % 8 == 0 && !((uintptr_t)x & 15) && !((uintptr_t)wt & 15);
+}
+
 extern "C" int iris_hip_vae_conv_out(uint8_t *rgb, float *f32, const uint16_t *g, int H, int W, int cin,
                                      const float *wt, const float *bias) {
-    if (!rgb || !g || !wt || !bias || H <= 0 || W <= 0 || H > 32768 || W > 32768 || cin <= 0 || cin > 256 || cin % 8 ||
-        ((uintptr_t)g & 15) ||
-        ((uintptr_t)wt & 15))
-        return iris_set_error("vae_conv_out: bad arguments");
-    if (cin % CO_C == 0) {
-        IRIS_LAUNCH(conv_out_tiled_kernel, dim3((W + CO_T - 1) / CO_T, (H + CO_T - 1) / CO_T), dim3(NT), 0,
-                    iris_stream(), g, H, W, cin, wt, bias, rgb, f32);
-        return iris_launch_check("conv_out_tiled_kernel");
-    }
-    const int npix = H * W;
-    IRIS_LAUNCH(conv_out_kernel, dim3((npix + NT - 1) / NT), dim3(NT), 9 * cin * sizeof(float4), iris_stream(),
-                       g, H, W, cin, wt, bias, rgb, f32);
-    return iris_launch_check("conv_out_kernel");
+    if (!conv_out_ok(rgb, g, H, W, cin, wt, bias)) return iris_set_error("vae_conv_out: bad arguments");
+    return launch_conv_out<uint16_t, false>(g, NULL, H, W, cin, wt, bias, rgb, f32);
+}
+
+extern "C" int iris_hip_vae_conv_out_norm(uint8_t *rgb, float *f32, const float *x, const float *ab, int H, int W,
+                                          int cin, const float *wt, const float *bias) {
+    if (!ab || !conv_out_ok(rgb, x, H, W, cin, wt, bias)) return iris_set_error("vae_conv_out_norm: bad arguments");
+    return launch_conv_out<float, true>(x, ab, H, W, cin, wt, bias, rgb, f32);
 }
 
 extern "C" int iris_hip_vae_img_in(uint16_t *out, const float *img, int H, int W) {

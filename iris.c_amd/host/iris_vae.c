@@ -506,13 +506,17 @@ oom:
     return fail("work buffers");
 }
 
-static int gn(iris_vae_gpu_t *v, const void *x, int is_bf16, int pix, int C, const float *g, const float *b,
-              int swish, uint16_t *y, uint16_t *raw) {
-    /* the sums from the producing convolution's epilogue, or a statistics pass */
+/* a GroupNorm's scale and shift of x into ab: from the sums of the producing
+ * convolution's epilogue, or a statistics pass */
+static int gn_ab(iris_vae_gpu_t *v, const void *x, int is_bf16, int pix, int C, const float *g, const float *b) {
     const int nblk = v->st_buf == x ? v->st_nblk : iris_hip_gn_stats(x, is_bf16, pix, C, VAE_GROUPS, v->part, GN_BLOCKS);
     v->st_buf = NULL;
-    if (nblk < 0 || iris_hip_gn_finalize(v->part, nblk, pix, C, VAE_GROUPS, g, b, v->eps, v->ab)) return -1;
-    return iris_hip_gn_apply(x, is_bf16, v->ab, pix, C, swish, y, raw);
+    return nblk < 0 || iris_hip_gn_finalize(v->part, nblk, pix, C, VAE_GROUPS, g, b, v->eps, v->ab) ? -1 : 0;
+}
+
+static int gn(iris_vae_gpu_t *v, const void *x, int is_bf16, int pix, int C, const float *g, const float *b,
+              int swish, uint16_t *y, uint16_t *raw) {
+    return gn_ab(v, x, is_bf16, pix, C, g, b) || iris_hip_gn_apply(x, is_bf16, v->ab, pix, C, swish, y, raw) ? -1 : 0;
 }
 
 /* stats: the output feeds a GroupNorm, so an unsplit convolution also forms
@@ -645,8 +649,8 @@ int iris_vae_gpu_decode_device(iris_vae_gpu_t *v, const float *d_lat, int lh, in
             W *= 2;
         }
     }
-    if (gn(v, v->x, 0, H * W, VAE_BASE, v->no_g, v->no_b, 1, v->t, NULL) ||
-        iris_hip_vae_conv_out(d_rgb, d_f32, v->t, H, W, VAE_BASE, v->co_w, v->co_b))
+    if (gn_ab(v, v->x, 0, H * W, VAE_BASE, v->no_g, v->no_b) ||
+        iris_hip_vae_conv_out_norm(d_rgb, d_f32, v->x, v->ab, H, W, VAE_BASE, v->co_w, v->co_b))
         return fail("decode (output)");
     return 0;
 }
