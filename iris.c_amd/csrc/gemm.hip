@@ -1837,7 +1837,7 @@ namespace {
  * behind a load each.
  *
  * 8 waves as in gemm_ring_kernel: waves 0..3 compute (2x2, wave tile 8 pixel
- * rows x 64 channels), waves 4..7 load, one barrier per K step (a tap of a
+ * rows x TN / 2 channels), waves 4..7 load, one barrier per K step (a tap of a
  * 64-channel chunk; taps within chunks). Weights go through 4 stages. The
  * patch has two buffers: chunk c+1's is loaded in the first AL steps of chunk
  * c, and it is complete when step 8 of chunk c waits for the weights of the
@@ -1862,18 +1862,18 @@ struct ConvParams {
     int gn_groups;
 };
 
-template <bool UP>
+template <bool UP, int TN>
 __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) {
     constexpr int PW = UP ? 10 : 18, NPX = PW * PW, SLOTS = (NPX + 7) / 8, AL = (SLOTS + 7) / 8;
-    constexpr int A_BYTES = SLOTS * 1024, W_BYTES = 128 * BK * 2, NSW = 4, FM_ = 8, FN_ = 4;
+    constexpr int A_BYTES = SLOTS * 1024, W_BYTES = TN * BK * 2, NSW = 4, FM_ = 8, FN_ = TN / 32, WL = TN / 32;
     extern __shared__ __attribute__((aligned(16))) char sm[];
-    __shared__ float gnl[16][32][2];
+    __shared__ float gnl[2048 / TN][TN / 4][2];
     const int L = (blockIdx.x & 7) * P.per_xcd + (blockIdx.x >> 3);
     if (L >= P.total) return;
     /* scalar registers for what the buffer resources and addresses are made of */
     const int split = __builtin_amdgcn_readfirstlane(L / P.tiles), Ls = L - split * P.tiles;
     const int tile = __builtin_amdgcn_readfirstlane(Ls / P.tn), ty = __builtin_amdgcn_readfirstlane(tile / P.tx);
-    const int n0 = (Ls - tile * P.tn) * 128, y0 = ty * 16, x0 = (tile - ty * P.tx) * 16;
+    const int n0 = (Ls - tile * P.tn) * TN, y0 = ty * 16, x0 = (tile - ty * P.tx) * 16;
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c0 = split * P.cps, chunks = min(P.cps, P.cin / BK - c0);   /* this block's 64-channel chunks */
@@ -1889,7 +1889,7 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
         const __amdgpu_buffer_rsrc_t a_rsrc =
             __builtin_amdgcn_make_buffer_rsrc((void *)P.in, (short)0, (int)P.in_bytes, 0x00020000);
         const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)(P.wt + (size_t)n0 * 9 * P.cin), (short)0, min(128, P.cout - n0) * 9 * P.cin * 2, 0x00020000);
+            (void *)(P.wt + (size_t)n0 * 9 * P.cin), (short)0, min(TN, P.cout - n0) * 9 * P.cin * 2, 0x00020000);
         /* patch slot j holds patch pixels 8j .. 8j+7; this wave's are
          * 8s + 2 lw + i of step s (the last slot again past the end). Pixels
          * outside the image, and past the patch, read as zero: an offset past
@@ -1907,7 +1907,7 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
         int w_off[2];
 #pragma unroll
         for (int par = 0; par < 2; par++)
-            w_off[par] = (lw * 32 + drow) * 9 * P.cin * 2 + ((dch ^ ((4 * par + (drow >> 1)) & 7)) << 4);
+            w_off[par] = (lw * (TN / 4) + drow) * 9 * P.cin * 2 + ((dch ^ ((4 * par + (drow >> 1)) & 7)) << 4);
         const int w_step = 8 * 9 * P.cin * 2;
         auto dma_a = [&](int chunk, int i) {
             const int slot = min((i >> 1) * 8 + lw * 2 + (i & 1), SLOTS - 1);
@@ -1918,8 +1918,8 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
         auto dma_w = [&](int stage, int chunk, int tap) {
             const int soff = (tap * P.cin + (c0 + chunk) * BK) * 2;
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(wring + stage * W_BYTES + (lw * 4 + i) * 1024),
+            for (int i = 0; i < WL; i++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(wring + stage * W_BYTES + (lw * WL + i) * 1024),
                                                          16, w_off[i & 1] + i * w_step, soff, 0, 0);
         };
 #pragma unroll
@@ -1927,7 +1927,7 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
 #pragma unroll
         for (int g = 0; g < NSW; g++) dma_w(g, 0, g);
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm((NSW - 1) * 4, 15));
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm((NSW - 1) * WL, 15));
         barrier();
         /* Step s waits for the weights of the next step: issued 3 steps ago,
          * before the loads of the last two. After the barrier it issues its
@@ -1936,7 +1936,7 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
 #define CONV_STEP(s)                                                                                               \
     do {                                                                                                           \
         __builtin_amdgcn_s_waitcnt(                                                                                \
-            waitcnt_imm(8 + (((s) + 8) % 9 < AL ? 2 : 0) + (((s) + 7) % 9 < AL ? 2 : 0), 15));                     \
+            waitcnt_imm(2 * WL + (((s) + 8) % 9 < AL ? 2 : 0) + (((s) + 7) % 9 < AL ? 2 : 0), 15));                     \
         barrier();                                                                                                 \
         if ((s) < AL) {                                                                                            \
             dma_a(chunk + 1, (s) < AL ? 2 * (s) : 0);                                                              \
@@ -1971,7 +1971,7 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
             const int c = UP ? ((lr + dx - 1) >> 1) + 1 : lr + dx;
             ab[dx][kk] = (wm * (UP ? 4 : 8) * PW + c) * 128 + (((kk * 4 + lg) ^ ((c >> 1) & 7)) << 4);
         }
-        wb[kk] = swz(wn * 64 + lr, kk * 4 + lg) * 2;
+        wb[kk] = swz(wn * (TN / 2) + lr, kk * 4 + lg) * 2;
     }
     bf16x8 a0[FM_], w0[FN_], a1[FM_], w1[FN_];
     auto frags = [&](int buf, int st, int s, int kk, bf16x8 (&a)[FM_], bf16x8 (&w)[FN_]) {
@@ -1995,7 +1995,7 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
 #pragma unroll
         for (int i = 0; i < FM_ + FN_; i++) {
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, FM_ * FN_ / (FM_ + FN_), 0);
         }
     };
     barrier();   /* chunk 0's patch, step 0's weights */
@@ -2018,24 +2018,24 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
     }
     }
 
-    /* The tile leaves through LDS (free now), as f32 rows of 128 channels and
-     * 16 bytes: all eight waves store it, 32 lanes a whole pixel row, and the
-     * residual is in flight meanwhile. Thread t has the 4 channels 4 (t % 32)
-     * of pixels t / 32 + 16 i. Pixels outside the image take an address inside
+    /* The tile leaves through LDS (free now), as f32 rows of TN channels and
+     * 16 bytes: all eight waves store it, TN / 4 lanes a whole pixel row, and the
+     * residual is in flight meanwhile. Thread t has the 4 channels 4 c4
+     * of pixels pr0 + OPX i. Pixels outside the image take an address inside
      * it and are not stored. */
-    constexpr int OSTR = 132;
+    constexpr int OSTR = TN + 4, OPX = 2048 / TN, ONI = 256 / OPX;
     static_assert(256 * OSTR * 4 <= 2 * A_BYTES + NSW * W_BYTES || UP, "the f32 tile fits the rings");
     float *const ot = (float *)sm;
-    const int c4 = tid & 31, pr0 = tid >> 5, col = n0 + c4 * 4;
+    const int c4 = tid & (TN / 4 - 1), pr0 = tid / (TN / 4), px = pr0 & 15, py = pr0 >> 4, col = n0 + c4 * 4;
     const bool part = P.ws != nullptr;   /* a split's partial sums: plain f32 rows of cout channels */
     void *const out = part ? (void *)(P.ws + split * P.ws_stride) : P.out;
     const int epi = part ? IRIS_EPI_F32 : P.epi, ldo = part ? P.cout : P.ldo;
     const float *const bias = part ? nullptr : P.bias;
-    size_t off[16];
-    float4 res[16];
+    size_t off[ONI];
+    float4 res[ONI];
 #pragma unroll
-    for (int i = 0; i < 16; i++) {   /* i: the tile's pixel row, pr0: its column */
-        off[i] = ((size_t)min(y0 + i, P.H - 1) * P.W + min(x0 + pr0, P.W - 1)) * ldo + col;
+    for (int i = 0; i < ONI; i++) {
+        off[i] = ((size_t)min(y0 + i * (OPX / 16) + py, P.H - 1) * P.W + min(x0 + px, P.W - 1)) * ldo + col;
         if (epi == IRIS_EPI_ADD) res[i] = *(const float4 *)((const float *)out + off[i]);
     }
     __syncthreads();   /* every read and every load of the rings is done */
@@ -2044,15 +2044,15 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
         for (int mi = 0; mi < FM_; mi++)
 #pragma unroll
             for (int ni = 0; ni < FN_; ni++)
-                *(f32x4 *)(ot + ((wm * 8 + mi) * 16 + lr) * OSTR + wn * 64 + ni * 16 + lg * 4) = acc[mi][ni];
+                *(f32x4 *)(ot + ((wm * 8 + mi) * 16 + lr) * OSTR + wn * (TN / 2) + ni * 16 + lg * 4) = acc[mi][ni];
     }
     __syncthreads();
     const float4 v = bias ? *(const float4 *)(bias + col) : make_float4(0, 0, 0, 0);
     float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const bool on = y0 + i < P.H && x0 + pr0 < P.W;
-        const float4 q = *(const float4 *)(ot + (i * 16 + pr0) * OSTR + c4 * 4);
+    for (int i = 0; i < ONI; i++) {
+        const bool on = y0 + i * (OPX / 16) + py < P.H && x0 + px < P.W;
+        const float4 q = *(const float4 *)(ot + (i * OPX + pr0) * OSTR + c4 * 4);
         float4 r = make_float4(q.x + v.x, q.y + v.y, q.z + v.z, q.w + v.w);
         if (epi == IRIS_EPI_ADD) {
             r.x += res[i].x; r.y += res[i].y; r.z += res[i].z; r.w += res[i].w;
@@ -2069,16 +2069,16 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
         }
     }
     if (gn) {
-        /* per thread the sums of 4 channels over 16 pixels, then the 16
+        /* per thread the sums of 4 channels over its pixels, then the OPX
          * threads of the channels and the group's chunks in order, in f64 */
         gnl[pr0][c4][0] = s1;
         gnl[pr0][c4][1] = s2;
         __syncthreads();
         const int cpg = P.cout / P.gn_groups;
-        if (tid < 128 / cpg) {
+        if (tid < TN / cpg) {
             double s = 0.0, q = 0.0;
             for (int c = tid * cpg / 4; c < (tid + 1) * cpg / 4; c++)
-                for (int m = 0; m < 16; m++) {
+                for (int m = 0; m < OPX; m++) {
                     s += (double)gnl[m][c][0];
                     q += (double)gnl[m][c][1];
                 }
@@ -2089,20 +2089,25 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
     }
 }
 
-template <bool UP> int launch_patch(const ConvParams &P) {
+template <bool UP, int TN> int launch_patch(const ConvParams &P) {
     constexpr int PW = UP ? 10 : 18;
     /* the rings, or the f32 tile of the epilogue */
-    constexpr size_t ring = 2 * ((PW * PW + 7) / 8) * 1024 + 4 * 128 * BK * 2, ot = 256 * 132 * 4;
+    constexpr size_t ring = 2 * ((PW * PW + 7) / 8) * 1024 + 4 * TN * BK * 2, ot = 256 * (TN + 4) * 4;
     constexpr size_t smem = ring > ot ? ring : ot;
     static std::once_flag once;
     static hipError_t attr = hipSuccess;
     std::call_once(once, [] {
-        attr = hipFuncSetAttribute((const void *)conv3x3_patch_kernel<UP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        attr = hipFuncSetAttribute((const void *)conv3x3_patch_kernel<UP, TN>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)smem);
     });
     if (iris_check(attr, "conv3x3 smem attribute")) return -1;
-    IRIS_LAUNCH((conv3x3_patch_kernel<UP>), dim3(8 * P.per_xcd), dim3(512), smem, iris_stream(), P);
+    IRIS_LAUNCH((conv3x3_patch_kernel<UP, TN>), dim3(8 * P.per_xcd), dim3(512), smem, iris_stream(), P);
     return iris_launch_check("conv3x3_patch_kernel");
+}
+
+int launch_patch_of(int up, int tn, const ConvParams &P) {
+    if (up) return tn == 64 ? launch_patch<true, 64>(P) : launch_patch<true, 128>(P);
+    return tn == 64 ? launch_patch<false, 64>(P) : launch_patch<false, 128>(P);
 }
 
 }  // namespace
@@ -2119,12 +2124,7 @@ extern "C" int iris_hip_conv3x3_tiled(const iris_conv3x3_t *c, int *gn_blocks) {
     const double area = (double)c->H * c->W;
     /* Tiles past one round may overshoot the image by a third (the products
      * of the overshoot cost time there; at 1.13, 90 x 166, they still win);
-     * within a round they only use idle CUs. Few tiles are split over the
-     * input channels by an estimate (us): 0.5 per K step, 8 per block, the
-     * partials written and read at 2.2 TB/s with one launch more, and a
-     * statistics pass where the sums were asked for: 64 x 64 pixels, 512 ->
-     * 512 (64 tiles) 56 us + 9 us of reduce pass in the 256-row kernel, split
-     * by 2 or 4 here 35. */
+     * within a round they only use idle CUs. */
     if (c->cout % 128 || c->ldo % 4 || (((uintptr_t)c->out | (uintptr_t)c->bias) & 15) || tiles >= (1LL << 28) ||
         (tiles > cus && 256.0 * ty * tx > 1.35 * area))
         return other();
@@ -2132,30 +2132,44 @@ extern "C" int iris_hip_conv3x3_tiled(const iris_conv3x3_t *c, int *gn_blocks) {
     if (conv_params(c, 128, chk)) return -1;
     const int chunks = c->cin / BK;
     const bool can = c->ws && !((uintptr_t)c->ws & 15);
-    int splits = 1;
+    /* Few tiles: half their channels each where twice as many still have a CU
+     * (a GroupNorm's group must stay within a tile), and a split over the
+     * input channels, by an estimate (us): 0.5 per K step of 128 channels, 0.3
+     * of 64, 8 per block, the partials written and read at 2.2 TB/s with one
+     * launch more, and a statistics pass where the sums were asked for.
+     * Measured, 128 channels / 64 / 64 split by 4: 64 x 64, 512 -> 512 (64
+     * tiles of 128) 44.4 / 30.8 / 42.7; 96 x 96, 256 -> 256 (72) 26.4 / 18.6 /
+     * 41.9; 64 x 128, 512 -> 512 (128) 46.5 / 38.0 / 73.5; 32 x 32, 512 -> 512
+     * (16) 40.3 / 26.3 / 25.2; past a CU per tile 64 lose: 128 x 128, 512 ->
+     * 512 (256) 59.3 / 70.8. */
+    const int groups = c->gn_part ? c->gn_groups : 0;
+    const bool can64 = !groups || (c->cout % groups == 0 && 64 % (c->cout / groups) == 0);
+    int splits = 1, tn = 128;
     double best = 1e30;
-    for (int s = 1; s <= 8 && s <= chunks; s *= 2) {
-        const double part = 4.0 * area * c->cout;
-        if (s > 1 && (!can || tiles * s > cus || s * part > (double)c->ws_bytes)) break;
-        const double us = 9.0 * ((chunks + s - 1) / s) * 0.5 + 8.0 +
-                          (s > 1 ? (s + 1) * part / 2.2e6 + 5.0 + (c->gn_part ? 7.0 : 0.0) : 0.0);
-        if (us < best) { best = us; splits = s; }
-    }
+    for (int n = 128; n >= (can64 ? 64 : 128); n /= 2)
+        for (int s = 1; s <= 8 && s <= chunks; s *= 2) {
+            const double part = 4.0 * area * c->cout;
+            if ((s > 1 || n < 128) && tiles * (128 / n) * s > cus) break;
+            if (s > 1 && (!can || s * part > (double)c->ws_bytes)) break;
+            const double us = 9.0 * ((chunks + s - 1) / s) * (n == 128 ? 0.5 : 0.3) + 8.0 +
+                              (s > 1 ? (s + 1) * part / 2.2e6 + 3.5 + (c->gn_part ? 3.5 : 0.0) : 0.0);
+            if (us < best) { best = us; splits = s; tn = n; }
+        }
     ConvParams P;
     memset(&P, 0, sizeof(P));
     P.in = c->in; P.wt = c->wt; P.out = c->out; P.bias = c->bias;
     P.H = c->H; P.W = c->W; P.cin = c->cin; P.cout = c->cout; P.ldo = c->ldo; P.epi = c->epi;
-    P.tx = (int)tx; P.tn = c->cout / 128; P.tiles = (int)tiles;
+    P.tx = (int)tx; P.tn = c->cout / tn; P.tiles = (int)(ty * tx * P.tn);
     P.cps = (chunks + splits - 1) / splits;
     P.total = P.tiles * splits; P.per_xcd = (P.total + 7) / 8;
     P.in_bytes = chk.conv_in_bytes;
     if (splits == 1) {
         P.gn_part = c->gn_part; P.gn_groups = c->gn_groups;
         if (gn_blocks && c->gn_part) *gn_blocks = (int)(ty * tx);
-        return c->up ? launch_patch<true>(P) : launch_patch<false>(P);
+        return launch_patch_of(c->up, tn, P);
     }
     P.ws = c->ws;
     P.ws_stride = (long long)c->H * c->W * c->cout;
-    if (c->up ? launch_patch<true>(P) : launch_patch<false>(P)) return -1;
+    if (launch_patch_of(c->up, tn, P)) return -1;
     return launch_reduce(&chk.p[0], &P.ws, &P.ws_stride, &splits, 1);
 }

@@ -121,3 +121,35 @@ def test_conv3x3_tiled_split(lib, H, W, cin, cout, up):
         assert split and np.array_equal(got[0], got[1])
         y = tl.bf16_to_f32(got[0]) if epi == EPI_BF16 else got[0]
         assert tl.rel_l2(y, ref + x0 if epi == EPI_ADD else ref) < (4e-3 if epi == EPI_BF16 else 1e-5)
+
+
+@pytest.mark.parametrize("H,W,cin,cout,up", [(64, 48, 256, 512, 0), (61, 50, 128, 256, 0), (33, 31, 512, 128, 0),
+                                             (64, 64, 128, 256, 1), (50, 34, 64, 128, 1)])
+def test_conv3x3_tiled_few_tiles(lib, H, W, cin, cout, up):
+    """Tiles of 64 channels (twice the tiles of 128 still have a CU each):
+    whole, ragged and upsampled, over one and several chunks."""
+    test_conv3x3_tiled(lib, H, W, cin, cout, up, True)
+
+
+@pytest.mark.parametrize("G", [8, 16, 32])
+def test_conv3x3_tiled_wide_groups(lib, G):
+    """Groups of 128, 64 and 32 channels: wider than, as wide as and within a
+    64-channel tile."""
+    H = W = 16
+    cin, cout = 64, 1024
+    rng = np.random.default_rng(G)
+    x = bf(rng.standard_normal((H, W, cin)).astype(np.float32))
+    w = bf((rng.standard_normal((cout, 9, cin)) / np.sqrt(9 * cin)).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    dx, dw, db = tl.Dev.of(tl.to_bf16(x)), tl.Dev.of(tl.to_bf16(w)), tl.Dev.of(b)
+    o, part = tl.Dev(H * W * cout * 4), tl.Dev(G * 16)
+    c = tl.Conv3x3(dx.ptr, dw.ptr, o.ptr, db.ptr, H, W, cin, cout, 0, cout, EPI_F32, 1, None, 0, part.ptr, G)
+    n = ctypes.c_int(-1)
+    assert lib.iris_hip_conv3x3_tiled(ctypes.byref(c), ctypes.byref(n)) == 0, lib.iris_hip_last_error()
+    assert n.value == 1
+    ref = conv64(x, w, b, 0)
+    assert tl.rel_l2(o.get(np.float32, (H, W, cout)), ref) < 1e-5
+    t = ref.reshape(H * W, G, cout // G)
+    # f32 sums of 64 to 128 values per thread, their rounding against the sum of magnitudes
+    np.testing.assert_allclose(part.get(np.float64, (G, 2)), np.stack([t.sum((0, 2)), (t * t).sum((0, 2))], -1),
+                               rtol=1e-4, atol=5e-2)
