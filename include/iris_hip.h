@@ -219,6 +219,10 @@ int iris_hip_conv3x3(const iris_conv3x3_t *c);
  * iris_hip_gn_finalize, at most ceil(H / 16) * ceil(W / 16) or
  * ceil(H * W / 256), or 0 if no sums were formed. */
 int iris_hip_conv3x3_tiled(const iris_conv3x3_t *c, int *gn_blocks);
+/* out (bf16, ldo == cout, 8-byte aligned) = c->out + the convolution: the
+ * epilogue IRIS_EPI_ADD (required) of a stream whose f32 sum nothing reads.
+ * c->out is undefined afterwards; no sums (gn_part NULL). */
+int iris_hip_conv3x3_add_bf16(const iris_conv3x3_t *c, uint16_t *d_out);
 
 /* ---- VAE decoder kernels (vae.hip), channels-last (NHWC) activations ---- */
 /* GroupNorm (iris_group_norm, iris_kernels.c:542) in three launches:

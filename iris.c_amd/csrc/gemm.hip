@@ -1860,6 +1860,7 @@ struct ConvParams {
     unsigned in_bytes;
     double *gn_part;
     int gn_groups;
+    uint16_t *bf16_out;   /* IRIS_EPI_ADD: the sum leaves here in bf16, out stays */
 };
 
 template <bool UP, int TN>
@@ -2029,6 +2030,8 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
     const int c4 = tid & (TN / 4 - 1), pr0 = tid / (TN / 4), px = pr0 & 15, py = pr0 >> 4, col = n0 + c4 * 4;
     const bool part = P.ws != nullptr;   /* a split's partial sums: plain f32 rows of cout channels */
     void *const out = part ? (void *)(P.ws + split * P.ws_stride) : P.out;
+    const bool to_bf16 = !part && (P.epi == IRIS_EPI_BF16 || P.bf16_out);
+    uint16_t *const out16 = P.bf16_out ? P.bf16_out : (uint16_t *)out;
     const int epi = part ? IRIS_EPI_F32 : P.epi, ldo = part ? P.cout : P.ldo;
     const float *const bias = part ? nullptr : P.bias;
     size_t off[ONI];
@@ -2058,8 +2061,8 @@ __global__ __launch_bounds__(512) void conv3x3_patch_kernel(const ConvParams P) 
             r.x += res[i].x; r.y += res[i].y; r.z += res[i].z; r.w += res[i].w;
         }
         if (on) {
-            if (epi == IRIS_EPI_BF16)
-                *(uint2 *)((uint16_t *)out + off[i]) =
+            if (to_bf16)
+                *(uint2 *)(out16 + off[i]) =
                     make_uint2((uint32_t)f2bf_hw(r.x) | ((uint32_t)f2bf_hw(r.y) << 16),
                                (uint32_t)f2bf_hw(r.z) | ((uint32_t)f2bf_hw(r.w) << 16));
             else
@@ -2112,11 +2115,18 @@ int launch_patch_of(int up, int tn, const ConvParams &P) {
 
 }  // namespace
 
-extern "C" int iris_hip_conv3x3_tiled(const iris_conv3x3_t *c, int *gn_blocks) {
+/* bf16_out (or NULL): the residual's sum in bf16 there, the f32 stream not
+ * written back (bound by bytes: 512 x 512 x 256 saves 134 MB and a pass of
+ * 400 MB; the 512 x 512 encode 1923 -> 1854 us, the 1024 x 1024 decode 11456
+ * -> 11347 with it in the blocks before a resampling) */
+static int conv_tiled(const iris_conv3x3_t *c, int *gn_blocks, uint16_t *bf16_out) {
     if (gn_blocks) *gn_blocks = 0;
+    auto convert = [&]() {
+        return bf16_out ? iris_hip_f32_to_bf16(bf16_out, (const float *)c->out, (size_t)c->H * c->W * c->cout) : 0;
+    };
     auto other = [&]() {
         if (gn_blocks && c && c->gn_part) *gn_blocks = (c->H * c->W + 255) / 256;
-        return iris_hip_conv3x3(c);
+        return iris_hip_conv3x3(c) ? -1 : convert();
     };
     if (!c || (c->up != 0 && c->up != 1) || c->H <= 0 || c->W <= 0 || c->cout <= 0 || c->splits > 1) return other();
     const int cus = iris_cu_count();
@@ -2166,10 +2176,21 @@ extern "C" int iris_hip_conv3x3_tiled(const iris_conv3x3_t *c, int *gn_blocks) {
     if (splits == 1) {
         P.gn_part = c->gn_part; P.gn_groups = c->gn_groups;
         if (gn_blocks && c->gn_part) *gn_blocks = (int)(ty * tx);
+        P.bf16_out = bf16_out;
         return launch_patch_of(c->up, tn, P);
     }
     P.ws = c->ws;
     P.ws_stride = (long long)c->H * c->W * c->cout;
     if (launch_patch_of(c->up, tn, P)) return -1;
-    return launch_reduce(&chk.p[0], &P.ws, &P.ws_stride, &splits, 1);
+    return launch_reduce(&chk.p[0], &P.ws, &P.ws_stride, &splits, 1) ? -1 : convert();
+}
+
+extern "C" int iris_hip_conv3x3_tiled(const iris_conv3x3_t *c, int *gn_blocks) {
+    return conv_tiled(c, gn_blocks, nullptr);
+}
+
+extern "C" int iris_hip_conv3x3_add_bf16(const iris_conv3x3_t *c, uint16_t *out) {
+    if (!c || !out || c->epi != IRIS_EPI_ADD || c->ldo != c->cout || c->gn_part || ((uintptr_t)out & 7))
+        return iris_set_error("conv3x3_add_bf16: bad arguments (a packed residual, no sums)");
+    return conv_tiled(c, nullptr, out);
 }

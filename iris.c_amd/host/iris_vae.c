@@ -521,8 +521,8 @@ static int gn(iris_vae_gpu_t *v, const void *x, int is_bf16, int pix, int C, con
 
 /* stats: the output feeds a GroupNorm, so an unsplit convolution also forms
  * its GroupNorm sums (cout / VAE_GROUPS channels per group) */
-static int conv(iris_vae_gpu_t *v, const uint16_t *in, const uint16_t *w, const float *b, void *out, int H, int W,
-                int cin, int cout, int up, int epi, int stats) {
+static int conv_to(iris_vae_gpu_t *v, const uint16_t *in, const uint16_t *w, const float *b, void *out, int H, int W,
+                   int cin, int cout, int up, int epi, int stats, uint16_t *bf16_out) {
     iris_conv3x3_t c;
     memset(&c, 0, sizeof(c));
     c.in = in;
@@ -553,12 +553,17 @@ static int conv(iris_vae_gpu_t *v, const uint16_t *in, const uint16_t *w, const 
     }
     v->st_buf = NULL;
     int nblk = 0;
-    if (iris_hip_conv3x3_tiled(&c, &nblk)) return -1;
+    if (bf16_out ? iris_hip_conv3x3_add_bf16(&c, bf16_out) : iris_hip_conv3x3_tiled(&c, &nblk)) return -1;
     if (nblk > 0) {
         v->st_buf = out;
         v->st_nblk = nblk;
     }
     return 0;
+}
+
+static int conv(iris_vae_gpu_t *v, const uint16_t *in, const uint16_t *w, const float *b, void *out, int H, int W,
+                int cin, int cout, int up, int epi, int stats) {
+    return conv_to(v, in, w, b, out, H, W, cin, cout, up, epi, stats, NULL);
 }
 
 static int gemm(iris_vae_gpu_t *v, const uint16_t *A, int lda, const uint16_t *W, int ldw, void *out, int ldo,
@@ -578,8 +583,10 @@ static void swap(float **a, float **b) {
 }
 
 /* resblock_forward (iris_vae.c:203-251): x += conv2(swish(gn2(conv1(swish(gn1(x)))))),
- * through a 1x1 shortcut into the other stream buffer when cin != cout */
-static int resblock(iris_vae_gpu_t *v, const vres_t *r, int H, int W) {
+ * through a 1x1 shortcut into the other stream buffer when cin != cout. last
+ * (or NULL): the sum in bf16 there instead of in x (resampled next, nothing
+ * else reads it) */
+static int resblock(iris_vae_gpu_t *v, const vres_t *r, int H, int W, uint16_t *last) {
     const int P = H * W;
     if (gn(v, v->x, 0, P, r->cin, r->n1g, r->n1b, 1, v->t, r->sk ? v->raw : NULL) ||
         conv(v, v->t, r->c1, r->c1b, v->h, H, W, r->cin, r->cout, 0, IRIS_EPI_BF16, 1) ||
@@ -587,12 +594,12 @@ static int resblock(iris_vae_gpu_t *v, const vres_t *r, int H, int W) {
         return -1;
     if (r->sk) {
         if (gemm(v, v->raw, r->cin, r->sk, r->cin, v->y, r->cout, r->skb, P, r->cout, r->cin, IRIS_EPI_F32) ||
-            conv(v, v->t, r->c2, r->c2b, v->y, H, W, r->cout, r->cout, 0, IRIS_EPI_ADD, 1))
+            conv_to(v, v->t, r->c2, r->c2b, v->y, H, W, r->cout, r->cout, 0, IRIS_EPI_ADD, !last, last))
             return -1;
         swap(&v->x, &v->y);
         return 0;
     }
-    return conv(v, v->t, r->c2, r->c2b, v->x, H, W, r->cout, r->cout, 0, IRIS_EPI_ADD, 1);
+    return conv_to(v, v->t, r->c2, r->c2b, v->x, H, W, r->cout, r->cout, 0, IRIS_EPI_ADD, !last, last);
 }
 
 /* attnblock_forward (iris_vae.c:260-357): single head over the S pixels,
@@ -632,16 +639,15 @@ int iris_vae_gpu_decode_device(iris_vae_gpu_t *v, const float *d_lat, int lh, in
     int H = 2 * lh, W = 2 * lw;
     if (iris_hip_vae_front(v->front, d_lat, v->z, lh, lw, v->lsc, v->lsh, v->divide, v->pqw, v->pqb) ||
         conv(v, v->front, v->cin_w, v->cin_b, v->x, H, W, VAE_CIN_PAD, VAE_MID, 0, IRIS_EPI_F32, 1) ||
-        resblock(v, &v->mid1, H, W) || attention(v, &v->attn, H, W) || resblock(v, &v->mid2, H, W))
+        resblock(v, &v->mid1, H, W, NULL) || attention(v, &v->attn, H, W) || resblock(v, &v->mid2, H, W, NULL))
         return fail("decode (mid block)");
     for (int level = 3, bi = 0; level >= 0; level--) {
         const int ch = VAE_BASE * ch_mult[level];
         for (int r = 0; r < 3; r++)
-            if (resblock(v, &v->up[bi++], H, W)) return fail("decode (resblock)");
+            if (resblock(v, &v->up[bi++], H, W, r == 2 && level > 0 ? v->raw : NULL)) return fail("decode (resblock)");
         if (level > 0) {
             /* nearest 2x + conv: the conv reads the bf16 stream through the upsample */
-            if (iris_hip_f32_to_bf16(v->raw, v->x, (size_t)H * W * ch) ||
-                conv(v, v->raw, v->ups_w[3 - level], v->ups_b[3 - level], v->y, 2 * H, 2 * W, ch, ch, 1,
+            if (conv(v, v->raw, v->ups_w[3 - level], v->ups_b[3 - level], v->y, 2 * H, 2 * W, ch, ch, 1,
                      IRIS_EPI_F32, 1))
                 return fail("decode (upsample)");
             swap(&v->x, &v->y);
@@ -713,18 +719,17 @@ int iris_vae_gpu_encode_device(iris_vae_gpu_t *v, const float *d_img, int H, int
     for (int level = 0, bi = 0; level < 4; level++) {
         const int ch = VAE_BASE * ch_mult[level];
         for (int r = 0; r < 2; r++)
-            if (resblock(v, &v->e_down[bi++], h, w)) return fail("encode (resblock)");
+            if (resblock(v, &v->e_down[bi++], h, w, r == 1 && level < 3 ? v->raw : NULL)) return fail("encode (resblock)");
         if (level < 3) {
             /* pad right/bottom + 3x3 stride 2, in the conv's loads */
-            if (iris_hip_f32_to_bf16(v->raw, v->x, (size_t)h * w * ch) ||
-                conv(v, v->raw, v->e_ds_w[level], v->e_ds_b[level], v->y, h / 2, w / 2, ch, ch, 2, IRIS_EPI_F32, 1))
+            if (conv(v, v->raw, v->e_ds_w[level], v->e_ds_b[level], v->y, h / 2, w / 2, ch, ch, 2, IRIS_EPI_F32, 1))
                 return fail("encode (downsample)");
             swap(&v->x, &v->y);
             h /= 2;
             w /= 2;
         }
     }
-    if (resblock(v, &v->e_mid1, h, w) || attention(v, &v->e_attn, h, w) || resblock(v, &v->e_mid2, h, w) ||
+    if (resblock(v, &v->e_mid1, h, w, NULL) || attention(v, &v->e_attn, h, w) || resblock(v, &v->e_mid2, h, w, NULL) ||
         gn(v, v->x, 0, h * w, VAE_MID, v->e_no_g, v->e_no_b, 1, v->t, NULL) ||
         conv(v, v->t, v->e_co_w, v->e_co_b, v->y, h, w, VAE_MID, 2 * v->z, 0, IRIS_EPI_F32, 0) ||
         iris_hip_vae_enc_out(d_lat, v->y, v->z, h, w, v->qw, v->qb, v->esc, v->esh))

@@ -153,3 +153,39 @@ def test_conv3x3_tiled_wide_groups(lib, G):
     # f32 sums of 64 to 128 values per thread, their rounding against the sum of magnitudes
     np.testing.assert_allclose(part.get(np.float64, (G, 2)), np.stack([t.sum((0, 2)), (t * t).sum((0, 2))], -1),
                                rtol=1e-4, atol=5e-2)
+
+
+@pytest.mark.parametrize("H,W,cin,cout,up,split", [
+    (173, 190, 128, 128, 0, False),   # 128-channel tiles, ragged
+    (61, 50, 128, 256, 0, False),     # 64-channel tiles
+    (64, 64, 128, 256, 1, False),     # through the upsample
+    (32, 32, 512, 512, 0, True),      # partial sums, then the conversion
+    (20, 23, 64, 192, 0, False),      # the other kernel, then the conversion
+])
+def test_conv3x3_add_bf16(lib, H, W, cin, cout, up, split):
+    """The residual epilogue leaving in bf16: the bits of IRIS_EPI_ADD followed
+    by the conversion."""
+    lib.iris_hip_conv3x3_add_bf16.argtypes = [ctypes.c_void_p] * 2
+    lib.iris_hip_f32_to_bf16.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t]
+    rng = np.random.default_rng(H + cin)
+    dx = tl.Dev.of(tl.to_bf16(rng.standard_normal((H >> up, W >> up, cin)).astype(np.float32)))
+    dw = tl.Dev.of(tl.to_bf16((rng.standard_normal((cout, 9, cin)) / np.sqrt(9 * cin)).astype(np.float32)))
+    db = tl.Dev.of(rng.standard_normal(cout).astype(np.float32))
+    x0 = rng.standard_normal((H, W, cout)).astype(np.float32)
+    nb = 8 * H * W * cout * 4
+    ws = tl.Dev(nb) if split else None
+    got = []
+    for direct in (True, False):
+        o, y = tl.Dev.of(x0), tl.Dev.of(np.zeros((H, W, cout), np.uint16))
+        c = tl.Conv3x3(dx.ptr, dw.ptr, o.ptr, db.ptr, H, W, cin, cout, up, cout, EPI_ADD, 0, ws.ptr if split else None,
+                       nb if split else 0, None, 0)
+        if direct:
+            assert lib.iris_hip_conv3x3_add_bf16(ctypes.byref(c), y.ptr) == 0, lib.iris_hip_last_error()
+        else:
+            assert lib.iris_hip_conv3x3_tiled(ctypes.byref(c), None) == 0, lib.iris_hip_last_error()
+            assert lib.iris_hip_f32_to_bf16(y.ptr, o.ptr, H * W * cout) == 0
+        assert lib.iris_hip_sync() == 0
+        got.append(y.get(np.uint16, (H, W, cout)))
+    assert np.array_equal(got[0], got[1]) and tl.bf16_to_f32(got[0]).std() > 0.5
+    c.epi = EPI_F32
+    assert lib.iris_hip_conv3x3_add_bf16(ctypes.byref(c), y.ptr) != 0
