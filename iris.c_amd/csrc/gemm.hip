@@ -1783,7 +1783,13 @@ extern "C" int iris_hip_conv3x3(const iris_conv3x3_t *c) {
     if (conv_params(c, 0, P)) return -1;
     const iris_gemm_problem_t &p = P.p[0];
     if (p.N <= 0) return 0;
-    const int bnt = p.N <= 128 ? 128 : BN;
+    /* 128 channels per tile also where 256 leave half the CUs without one (a
+     * GroupNorm's group must stay within a tile): 128 x 128 pixels out, stride
+     * 2, 256 -> 256 (64 tiles of 256) 62 -> 42 us; 64 x 64, 512 -> 512 split by
+     * 4 (128) 39 -> 30. */
+    const bool few = 2LL * P.tiles_m[0] * P.tiles_n[0] * (c->splits > 1 ? c->splits : 1) <= iris_cu_count();
+    const int bnt = p.N <= 128 || (few && (!c->gn_part || 128 % (p.N / c->gn_groups) == 0)) ? 128 : BN;
+    if (few && conv_params(c, bnt, P)) return -1;
     int chunks = 1;
     long long stride = 0;
     P.chunks[0] = 1;

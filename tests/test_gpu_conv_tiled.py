@@ -189,3 +189,35 @@ def test_conv3x3_add_bf16(lib, H, W, cin, cout, up, split):
     assert np.array_equal(got[0], got[1]) and tl.bf16_to_f32(got[0]).std() > 0.5
     c.epi = EPI_F32
     assert lib.iris_hip_conv3x3_add_bf16(ctypes.byref(c), y.ptr) != 0
+
+
+@pytest.mark.parametrize("H,W,cin,cout,up,G", [(17, 33, 64, 256, 2, 32), (16, 16, 128, 384, 2, 0), (20, 21, 64, 320, 0, 0),
+                                               (16, 32, 64, 256, 1, 2), (16, 16, 64, 512, 2, 2)])
+def test_conv3x3_narrow_tiles(lib, H, W, cin, cout, up, G):
+    """The implicit GEMM with few tiles: 128 channels each (a part-empty last
+    one too), 256 where a GroupNorm's group is wider; float64 outputs and sums."""
+    lib.iris_hip_conv3x3.argtypes = [ctypes.c_void_p]
+    rng = np.random.default_rng(H + cout)
+    shape = (2 * H, 2 * W, cin) if up == 2 else (H >> up, W >> up, cin)
+    x = bf(rng.standard_normal(shape).astype(np.float32))
+    w = bf((rng.standard_normal((cout, 9, cin)) / np.sqrt(9 * cin)).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    if up == 2:   # one row and column of zeros after the image, stride 2
+        ref = conv64(np.pad(x, ((0, 1), (0, 1), (0, 0))), w, b, 0)[1:-1:2, 1:-1:2]
+    else:
+        ref = conv64(x, w, b, up)
+    blocks = -(-H * W // 256)
+    dx, dw, db = tl.Dev.of(tl.to_bf16(x)), tl.Dev.of(tl.to_bf16(w)), tl.Dev.of(b)
+    o, part = tl.Dev(H * W * cout * 4), tl.Dev(blocks * max(G, 1) * 16)
+    c = tl.Conv3x3(dx.ptr, dw.ptr, o.ptr, db.ptr, H, W, cin, cout, up, cout, EPI_F32, 1, None, 0,
+                   part.ptr if G else None, G)
+    assert lib.iris_hip_conv3x3(ctypes.byref(c)) == 0, lib.iris_hip_last_error()
+    assert lib.iris_hip_sync() == 0
+    assert tl.rel_l2(o.get(np.float32, (H, W, cout)), ref) < 1e-5
+    if G:
+        pad = np.zeros((blocks * 256, cout))
+        pad[:H * W] = ref.reshape(-1, cout)
+        t = pad.reshape(blocks, 256, G, cout // G)
+        # f32 sums of 16 values, their rounding against the sum of magnitudes
+        np.testing.assert_allclose(part.get(np.float64, (blocks, G, 2)),
+                                   np.stack([t.sum((1, 3)), (t * t).sum((1, 3))], -1), rtol=1e-4, atol=5e-2)
