@@ -141,7 +141,8 @@ __global__ __launch_bounds__(NT) void gn_finalize_kernel(const double *part, int
  * HBM-bound once its arithmetic is short: the channel of a chunk by a mask (a
  * 64-bit remainder for channel counts that are no power of two), the hardware
  * reciprocal and bf16 conversion on values rounded to bf16 next. 1024 x 1024 x 128 bf16:
- * 129 -> 102 us (5.3 TB/s); f32 in 196 us (4.1 TB/s) before and after. */
+ * 129 -> 102 us (5.3 TB/s); f32 in 152-164 (4.9-5.3 TB/s); four 16-byte loads
+ * in flight per thread gave nothing more. */
 template <typename T>
 __global__ __launch_bounds__(NT) void gn_apply_kernel(const T *x, const float *ab, int C, size_t n8, int swish,
                                                       uint16_t *y, uint16_t *raw) {

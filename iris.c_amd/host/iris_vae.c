@@ -8,11 +8,12 @@
  *          -> mid: resblock, attention, resblock
  *          -> up levels 3..0: 3 resblocks, then nearest 2x + conv 3x3
  *             (levels 3..1; the upsample is folded into the conv's loads)
- *          -> GroupNorm + swish -> conv_out 128 -> 3 -> uint8 RGB.
- * The residual stream x is f32 [pixels][C]; GroupNorm writes the bf16 input
- * of each convolution; convolutions accumulate in f32 and add into x in their
- * epilogue. resblock_forward (iris_vae.c:203-251) and attnblock_forward
- * (iris_vae.c:260-357) map to resblock() and attention() below.
+ *          -> GroupNorm + swish -> conv_out 128 -> 3 -> uint8 RGB (one kernel).
+ * The residual stream x is f32 [pixels][C] (bf16 where a resampling follows);
+ * GroupNorm writes the bf16 input of each convolution; convolutions accumulate
+ * in f32 and add into x in their epilogue. resblock_forward
+ * (iris_vae.c:203-251) and attnblock_forward (iris_vae.c:260-357) map to
+ * resblock() and attention() below.
  */
 #include "../../include/iris_vae.h"
 #include "../../include/iris_hip.h"
