@@ -133,7 +133,8 @@ int iris_hip_gemm_splitk(const iris_gemm_problem_t *problem, int splits, float *
  * of 64: up to CUs / tiles chunks of at least 4 steps, as many as the
  * workspace holds (splits * M * N floats); otherwise the plain launch. For
  * the products on few rows (a 512-token caption or text stream, a 128-column
- * final projection) that leave most of the chip idle. */
+ * final projection) that leave most of the chip idle. Products of at most 128
+ * rows take iris_hip_gemm_ring's kernel. */
 int iris_hip_gemm_fill(const iris_gemm_problem_t *problem, float *d_workspace, size_t workspace_bytes);
 
 /* No counterpart in the reference. iris_hip_gemm_fill over up to 4

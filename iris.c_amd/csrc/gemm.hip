@@ -13,9 +13,11 @@
  * a 4x2 arrangement; each wave owns 64x128 as 4x8 v_mfma_f32_16x16x32_bf16
  * tiles (narrower block tiles: 256x224 for plain GEMMs whose last round of
  * 256-wide tiles would be part-empty, 256x128 for convolutions of at most
- * 128 output channels). The 16x16x32 form does the same work per LDS byte as 32x32x16 and,
- * with the chip at its power limit on random data, sustains about 10 % more
- * MFMA throughput.
+ * 128 output channels or few tiles). The 16x16x32 form does the same work per
+ * LDS byte as 32x32x16 and, with the chip at its power limit on random data,
+ * sustains about 10 % more MFMA throughput. Products of few rows run on
+ * gemm_ring_kernel and most stride-1 convolutions on conv3x3_patch_kernel,
+ * both below.
  *
  * Waves w and w+4 share a SIMD. The two groups (waves 0..3, waves 4..7) run
  * ping-pong: separated by block barriers, one group reads a whole 64-wide K

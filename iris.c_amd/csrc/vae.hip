@@ -344,7 +344,7 @@ __global__ __launch_bounds__(NT) void transpose_bf16_kernel(const uint16_t *src,
  * within an XCD's band, so a halo's second reading finds its L2.
  * Bound by its products (64 f32 MFMAs per 16 pixels, halo 1.2 times) with the
  * activation beside them: 1024 x 1024 x 128 in 187 us from f32, which replaces
- * an apply pass of 196-212 and a kernel of one thread per output over
+ * an apply pass of about 155 and a kernel of one thread per output over
  * LDS-staged tiles of 356; from bf16 about 180. */
 constexpr int CO_X = 30, CO_Y = 16, CO_W = CO_X + 2, CO_P = CO_W * (CO_Y + 2), CO_N = 27, CO_KC = 128;
 constexpr int CO_GW = CO_P / 16 / (NT / IRIS_WAVE);   /* groups of 16 pixels per wave */
