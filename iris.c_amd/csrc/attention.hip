@@ -72,9 +72,10 @@
  * wave per SIMD, the softmax of a tile under the QK products of the next.
  *
  * The Q prologue is VALU work (4 clocks an instruction per wave), so it uses
- * the hardware reciprocal square root and bf16 conversion and picks the
- * weight set once per wave: 3 to 4 us less per round of blocks (768 queries,
- * 72 units 28.1 -> 25.0 us; 4608, two rounds, 252.8 -> 247.1 us).
+ * the hardware bf16 conversion and picks the weight set once per wave: 1536 queries (144 units, one round) 51.8 ->
+ * 49.4 us, 4608 (two rounds) 269.8 -> 262.9.
+ * Square root and division stay correctly rounded and the rotation's fused
+ * products are written out, so a row has the bits of iris_hip_qk_prepare's.
  *
  * Blocks are ordered head-major and mapped XCD-major (block b runs on XCD
  * b % 8 and takes a contiguous range of the work list), so the query blocks
@@ -297,7 +298,7 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
 #pragma unroll
             for (int j = 0; j < 8; j++) { x[j] = bf2f(raw[pass][j]); ss += x[j] * x[j]; }
             ss = row16_sum(ss);
-            const float inv = __builtin_amdgcn_rsqf(ss * (1.0f / 128.0f) + a.qn_eps);
+            const float inv = 1.0f / sqrtf(ss / 128.0f + a.qn_eps);
             if (mixed && row >= a.qn_split) { ww0 = wb0; ww1 = wb1; }
             const float ww[8] = {ww0.x, ww0.y, ww0.z, ww0.w, ww1.x, ww1.y, ww1.z, ww1.w};
             const float c[4] = {c4[pass].x, c4[pass].y, c4[pass].z, c4[pass].w};
@@ -306,8 +307,8 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
 #pragma unroll
             for (int j = 0; j < 8; j += 2) {
                 const float x0 = x[j] * inv * ww[j], x1 = x[j + 1] * inv * ww[j + 1];
-                out[j] = f2bf_hw(x0 * c[j >> 1] - x1 * sn[j >> 1]);
-                out[j + 1] = f2bf_hw(x1 * c[j >> 1] + x0 * sn[j >> 1]);
+                out[j] = f2bf_hw(__builtin_fmaf(x0, c[j >> 1], -(x1 * sn[j >> 1])));
+                out[j + 1] = f2bf_hw(__builtin_fmaf(x0, sn[j >> 1], x1 * c[j >> 1]));
             }
             *(u16x8 *)(qs + rw * KSTR + d0) = out;
         }
@@ -736,10 +737,11 @@ extern "C" int iris_hip_attention(const iris_attn_args_t *a) {
     }
     /* 128 queries per block (4 waves) where those blocks still fit one round:
      * twice the CUs at work, and half the prologue per CU. Same bits. Measured,
-     * us, 8 waves -> 4 (24 heads, keys = queries): 768 25.0 -> 20.7, 1024 31.4
-     * -> 26.6, 1280 37.1 -> 31.6; 32 heads causal: 37 11.1 -> 7.9, 512 26.0 ->
-     * 17.9. Past one round the second one costs more: 1536 (288 blocks) 42.0
-     * -> 65.6, and at 4608 the two groups' overlap wins, 247 -> 345. */
+     * us between events, 8 waves -> 4 (24 heads, keys = queries): 512 22.3 ->
+     * 18.6, 768 28.4 -> 23.8, 1024 35.1 -> 29.9, 1280 42.1 -> 36.0; 32 heads
+     * causal: 37 14.5 -> 11.1, 512 30.4 -> 21.4. Past one round the second
+     * one costs more: 1536 (288 blocks) 42.0 -> 65.6, and at 4608 the two
+     * groups' overlap wins, 247 -> 345. */
     const int nqb4 = (a->sq + 4 * QW - 1) / (4 * QW);
     const long long total4 = (long long)nqb4 * a->heads * a->batch;
     if (total4 <= cus) {

@@ -279,13 +279,14 @@ __device__ __forceinline__ void qk_norm_rope_rows(const iris_qkprep_args_t &a, i
 #pragma unroll
             for (int j = 0; j < 8; j++) { x[j] = bf2f(raw[j]); ss += x[j] * x[j]; }
             ss = row16_sum(ss);
-            const float inv = __builtin_amdgcn_rsqf(ss * (1.0f / 128.0f) + a.eps);
+            const float inv = 1.0f / sqrtf(ss / 128.0f + a.eps);
             u16x8 out;
 #pragma unroll
             for (int j = 0; j < 8; j += 2) {
                 const float x0 = x[j] * inv * w[j], x1 = x[j + 1] * inv * w[j + 1];
-                out[j] = f2bf_hw(x0 * c[j] - x1 * sn[j]);
-                out[j + 1] = f2bf_hw(x1 * c[j] + x0 * sn[j]);
+                /* fused as written, as in the attention's Q prologue */
+                out[j] = f2bf_hw(__builtin_fmaf(x0, c[j], -(x1 * sn[j])));
+                out[j + 1] = f2bf_hw(__builtin_fmaf(x0, sn[j], x1 * c[j]));
             }
             if (on) *(u16x8 *)(dst + head * 128) = out;
         }
