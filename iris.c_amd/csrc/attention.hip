@@ -72,10 +72,10 @@
  * wave per SIMD, the softmax of a tile under the QK products of the next.
  *
  * The Q prologue is VALU work (4 clocks an instruction per wave), so it uses
- * the hardware bf16 conversion and picks the weight set once per wave: 1536 queries (144 units, one round) 51.8 ->
- * 49.4 us, 4608 (two rounds) 269.8 -> 262.9.
- * Square root and division stay correctly rounded and the rotation's fused
- * products are written out, so a row has the bits of iris_hip_qk_prepare's.
+ * the hardware bf16 conversion and picks the weight set once per wave: 1536
+ * queries (144 units, one round) 51.8 -> 49.4 us, 4608 (two rounds) 269.8 ->
+ * 262.9. Square root and division are correctly rounded and the rotation's
+ * fused products written out: a row has the bits of iris_hip_qk_prepare's.
  *
  * Blocks are ordered head-major and mapped XCD-major (block b runs on XCD
  * b % 8 and takes a contiguous range of the work list), so the query blocks

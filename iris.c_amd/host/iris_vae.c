@@ -468,12 +468,15 @@ static int score_rows(int S, int Kp) {
     return r < S ? r : S;
 }
 
-/* work buffers for an image of P = H*W pixels (S = P/64 bottleneck tokens) */
+/* work buffers for an image of P = H*W pixels (S = P/64 bottleneck tokens).
+ * ws_bytes is what this picture would have allocated, not what an earlier and
+ * larger one left: the plans split by it, and a picture's bits must not depend
+ * on the pictures before it */
 static int ensure_work(iris_vae_gpu_t *v, int lh, int lw) {
-    const size_t P = (size_t)256 * lh * lw;
+    const size_t P = (size_t)256 * lh * lw, S = P / 64, Kp = (S + 63) / 64 * 64;
+    v->ws_bytes = 4 * S * VAE_MID * sizeof(float);   /* split-K at the bottleneck */
     if (P <= v->cap_pix) return 0;
     free_work(v);
-    const size_t S = P / 64, Kp = (S + 63) / 64 * 64;
     /* score_rows keeps every later, smaller call within this many scores */
     const size_t n_sc = S * Kp < SCORE_ELEMS ? S * Kp : SCORE_ELEMS;
     ALLOC(v->x, P * 256 * sizeof(float));
@@ -494,7 +497,6 @@ static int ensure_work(iris_vae_gpu_t *v, int lh, int lw) {
     ALLOC(v->srow, S * 2 * sizeof(float));
     ALLOC(v->pm, n_sc * 2);
     ALLOC(v->front, S * VAE_CIN_PAD * 2);
-    v->ws_bytes = 4 * S * VAE_MID * sizeof(float);   /* split-K at the bottleneck */
     ALLOC(v->ws, v->ws_bytes);
     ALLOC(v->dlat, (size_t)v->lat_ch * lh * lw * sizeof(float));
     ALLOC(v->drgb, P * 3);

@@ -112,6 +112,26 @@ def test_image_api_and_determinism(lib, models):
     assert np.array_equal(data, rgb)
 
 
+@pytest.mark.parametrize("lh,lw", [(12, 12), (13, 12)])
+def test_bits_do_not_depend_on_earlier_pictures(lib, lh, lw):
+    """A small picture both ways on a fresh handle and after a large one has
+    grown the work buffers: the plans that split sums go by the picture."""
+    g = ctypes.c_void_p(lib.iris_vae_gpu_create_synthetic(32, 0.0, 0.0, 11))
+    assert g.value
+    img = np.random.default_rng(3).uniform(-1, 1, (3, 16 * lh, 16 * lw)).astype(np.float32)
+    dimg, dlat = tl.Dev.of(img), tl.Dev(128 * lh * lw * 4)
+
+    def both():
+        rgb, f32 = gpu_decode(lib, g, latent(32, lh, lw, 1))
+        assert lib.iris_vae_gpu_encode_device(g, dimg.ptr, 16 * lh, 16 * lw, dlat.ptr) == 0, lib.iris_hip_last_error()
+        return f32, dlat.get(np.float32, 128 * lh * lw)
+    first = both()
+    gpu_decode(lib, g, latent(32, 40, 40, 2))
+    again = both()
+    lib.iris_vae_gpu_free(g)
+    assert np.array_equal(first[0], again[0]) and np.array_equal(first[1], again[1])
+
+
 def test_load_dir_reads_config(lib, files, tmp_path):
     """vae/config.json selects z_channels and the Z-Image scaling branch
     (iris.c:332-392, iris_vae_config.h)."""
