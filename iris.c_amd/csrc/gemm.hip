@@ -2143,7 +2143,10 @@ static int conv_tiled(const iris_conv3x3_t *c, int *gn_blocks, uint16_t *bf16_ou
     /* Tiles past one round may overshoot the image by a third (the products
      * of the overshoot cost time there; at 1.13, 90 x 166, they still win);
      * within a round they only use idle CUs. */
-    if (c->cout % 128 || c->ldo % 4 || (((uintptr_t)c->out | (uintptr_t)c->bias) & 15) || tiles >= (1LL << 28) ||
+    /* a GroupNorm group wider than a tile, or no whole number of channels, is the other kernel's to take or refuse */
+    const int G = c->gn_part ? c->gn_groups : 0;
+    const bool wide = c->gn_part && (G <= 0 || c->cout % G || 128 % (c->cout / G));
+    if (c->cout % 128 || wide || c->ldo % 4 || (((uintptr_t)c->out | (uintptr_t)c->bias) & 15) || tiles >= (1LL << 28) ||
         (tiles > cus && 256.0 * ty * tx > 1.35 * area))
         return other();
     GemmParams chk;
@@ -2160,8 +2163,7 @@ static int conv_tiled(const iris_conv3x3_t *c, int *gn_blocks, uint16_t *bf16_ou
      * 41.9; 64 x 128, 512 -> 512 (128) 46.5 / 38.0 / 73.5; 32 x 32, 512 -> 512
      * (16) 40.3 / 26.3 / 25.2; past a CU per tile 64 lose: 128 x 128, 512 ->
      * 512 (256) 59.3 / 70.8. */
-    const int groups = c->gn_part ? c->gn_groups : 0;
-    const bool can64 = !groups || (c->cout % groups == 0 && 64 % (c->cout / groups) == 0);
+    const bool can64 = !G || 64 % (c->cout / G) == 0;
     int splits = 1, tn = 128;
     double best = 1e30;
     for (int n = 128; n >= (can64 ? 64 : 128); n /= 2)

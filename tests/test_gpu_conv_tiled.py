@@ -155,6 +155,28 @@ def test_conv3x3_tiled_wide_groups(lib, G):
                                rtol=1e-4, atol=5e-2)
 
 
+@pytest.mark.parametrize("cout,G,ok", [(1024, 4, True), (512, 2, True), (512, 1, False), (512, 3, False), (384, 2, False)])
+def test_conv3x3_tiled_groups_of_the_other_kernel(lib, cout, G, ok):
+    """Groups wider than a tile's 128 channels run on, or are refused by, the
+    other kernel, with its bits and sums and the number of its row tiles."""
+    H, W, cin = 20, 15, 64
+    rng = np.random.default_rng(G)
+    x = rng.standard_normal((H, W, cin)).astype(np.float32)
+    w = (rng.standard_normal((cout, 9, cin)) / np.sqrt(9 * cin)).astype(np.float32)
+    dx, dw = tl.Dev.of(tl.to_bf16(x)), tl.Dev.of(tl.to_bf16(w))
+    got = []
+    for tiled in (0, 1):
+        o, part = tl.Dev.of(np.zeros((H, W, cout), np.float32)), tl.Dev.of(np.zeros((2, G, 2)))
+        c = tl.Conv3x3(dx.ptr, dw.ptr, o.ptr, None, H, W, cin, cout, 0, cout, EPI_F32, 1, None, 0, part.ptr, G)
+        n = ctypes.c_int(-1)
+        rc = lib.iris_hip_conv3x3_tiled(ctypes.byref(c), ctypes.byref(n)) if tiled else lib.iris_hip_conv3x3(ctypes.byref(c))
+        assert (rc == 0) == ok, (tiled, lib.iris_hip_last_error())
+        if tiled and ok:
+            assert n.value == 2
+        got.append((o.get(np.uint32, (H, W, cout)), part.get(np.uint64, (2, G, 2))))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("H,W,cin,cout,up,split", [
     (173, 190, 128, 128, 0, False),   # 128-channel tiles, ragged
     (61, 50, 128, 256, 0, False),     # 64-channel tiles
