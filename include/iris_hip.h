@@ -38,8 +38,10 @@ int iris_hip_memcpy_d2h(void *dst, const void *d_src, size_t bytes);   /* synchr
 /* Download beside later work of the library stream: pinned memory of the
  * caller's, and a copy into it on the side stream, ordered after everything
  * enqueued on the library stream so far; iris_hip_download_wait returns when
- * the copy of that slot (0..7) is done. d_src is not rewritten before that.
- * Not for captured work. */
+ * the last copy of that slot (0..7) is done. The caller neither rewrites d_src
+ * nor frees or reads the pinned memory before that, also where it gives up
+ * half-way: iris_hip_sync waits for the library stream only. A download that
+ * returns an error leaves no copy behind. Not for captured work. */
 void *iris_hip_host_malloc(size_t bytes);            /* NULL on failure */
 void iris_hip_host_free(void *ptr);
 int iris_hip_download(void *pinned_dst, const void *d_src, size_t bytes, int slot);

@@ -21,6 +21,10 @@ static hipStream_t g_stream = nullptr;
  * fork / join order it against the library stream with two events */
 static hipStream_t g_side = nullptr;
 static hipEvent_t g_fork_ev = nullptr, g_join_ev = nullptr;
+/* iris_hip_download: order after the library stream, then behind each slot's copy */
+constexpr int DOWN_SLOTS = 8;
+static hipEvent_t g_down_at = nullptr, g_down_ev[DOWN_SLOTS];
+static bool g_down_used[DOWN_SLOTS];
 static int g_on_side = 0;
 static char g_err[512] = "";
 static char g_name[256] = "";
@@ -69,8 +73,11 @@ int iris_hip_init(int device) {
     /* both streams at the default priority */
     if (iris_check(hipStreamCreateWithFlags(&g_side, hipStreamNonBlocking), "hipStreamCreate (side)") ||
         iris_check(hipEventCreateWithFlags(&g_fork_ev, hipEventDisableTiming), "hipEventCreate (fork)") ||
-        iris_check(hipEventCreateWithFlags(&g_join_ev, hipEventDisableTiming), "hipEventCreate (join)"))
+        iris_check(hipEventCreateWithFlags(&g_join_ev, hipEventDisableTiming), "hipEventCreate (join)") ||
+        iris_check(hipEventCreateWithFlags(&g_down_at, hipEventDisableTiming), "hipEventCreate (download)"))
         return -1;
+    for (hipEvent_t &e : g_down_ev)
+        if (iris_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate (download)")) return -1;
     g_cus = p.multiProcessorCount;
     g_device = device;
     g_init = 1;
@@ -222,23 +229,23 @@ void iris_hip_host_free(void *p) {
     if (p) (void)hipHostFree(p);
 }
 
-/* events behind the copies of iris_hip_download, made on first use */
-static hipEvent_t g_down_ev[8], g_down_at;
-
 int iris_hip_download(void *dst, const void *src, size_t bytes, int slot) {
-    if (slot < 0 || slot >= 8 || !iris_hip_available()) return iris_set_error("download slot %d", slot);
-    if (!g_down_at && iris_check(hipEventCreateWithFlags(&g_down_at, hipEventDisableTiming), "download event")) return -1;
-    if (!g_down_ev[slot] &&
-        iris_check(hipEventCreateWithFlags(&g_down_ev[slot], hipEventDisableTiming), "download event"))
+    if (slot < 0 || slot >= DOWN_SLOTS || !dst || !src || !iris_hip_available())
+        return iris_set_error("download slot %d", slot);
+    if (iris_check(hipEventRecord(g_down_at, g_stream), "download order") ||
+        iris_check(hipStreamWaitEvent(g_side, g_down_at, 0), "download order") ||
+        iris_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g_side), "download"))
         return -1;
-    return iris_check(hipEventRecord(g_down_at, g_stream), "download order") ||
-           iris_check(hipStreamWaitEvent(g_side, g_down_at, 0), "download order") ||
-           iris_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g_side), "download") ||
-           iris_check(hipEventRecord(g_down_ev[slot], g_side), "download event");
+    if (iris_check(hipEventRecord(g_down_ev[slot], g_side), "download event")) {
+        (void)hipStreamSynchronize(g_side);   /* a refused download leaves no copy behind */
+        return -1;
+    }
+    g_down_used[slot] = true;
+    return 0;
 }
 
 int iris_hip_download_wait(int slot) {
-    if (slot < 0 || slot >= 8 || !g_down_ev[slot]) return iris_set_error("download slot %d", slot);
+    if (slot < 0 || slot >= DOWN_SLOTS || !g_down_used[slot]) return iris_set_error("download slot %d", slot);
     return iris_check(hipEventSynchronize(g_down_ev[slot]), "download wait");
 }
 

@@ -450,6 +450,16 @@ static int layer_forward(qwen3_model_t *m, const qlayer_t *l, const float *next_
     return 0;
 }
 
+/* waits for the downloads in flight (one bit per slot): they write the
+ * model's pinned memory from out, which the next call rewrites, so no exit
+ * leaves one behind */
+static int finish_downloads(unsigned slots) {
+    int rc = 0;
+    for (int s = 0; slots >> s; s++)
+        if ((slots >> s & 1) && iris_hip_download_wait(s)) rc = -1;
+    return rc;
+}
+
 float *qwen3_forward(qwen3_model_t *m, const int *input_ids, const int *attention_mask, int seq_len) {
     if (!m || !input_ids || seq_len < 1 || seq_len > QWEN3_MAX_SEQ_LEN) {
         fprintf(stderr, "qwen3_forward: seq_len %d outside [1, %d]\n", seq_len, QWEN3_MAX_SEQ_LEN);
@@ -486,25 +496,30 @@ float *qwen3_forward(qwen3_model_t *m, const int *input_ids, const int *attentio
     /* a small result is not worth the second stream's events (37 tokens, 379
      * KB: 2810 us with one copy at the end, 2932 with them) */
     const int beside = slots * n * sizeof(float) >= ((size_t)1 << 20);
+    unsigned sent = 0;   /* slots whose download is in flight */
     const iris_norm_args_t first = rms(m, m->L[0].ln1, S);
     if (iris_hip_rownorm(&first)) {
         fail("input norm");
         return NULL;
     }
     for (int i = 0; i <= last; i++) {
-        if (layer_forward(m, &m->L[i], i < last ? m->L[i + 1].ln1 : NULL, S, n_real)) return NULL;
+        if (layer_forward(m, &m->L[i], i < last ? m->L[i + 1].ln1 : NULL, S, n_real)) {
+            finish_downloads(sent);
+            return NULL;
+        }
         int slot = -1;
         if (m->mode) slot = i == last ? 0 : -1;
         else slot = i == QWEN3_OUTPUT_LAYER_1 ? 0 : i == QWEN3_OUTPUT_LAYER_2 ? 1 : i == QWEN3_OUTPUT_LAYER_3 ? 2 : -1;
         /* an extracted layer is copied aside and downloaded while the layers
          * after it run */
-        if (slot >= 0 && (iris_hip_copy_rows(m->out + slot * n, h, m->x, h, S, h) ||
-                          (beside && iris_hip_download(m->host_out + slot * n, m->out + slot * n, n * sizeof(float),
-                                                       slot)))) {
+        if (slot < 0) continue;
+        if (iris_hip_copy_rows(m->out + slot * n, h, m->x, h, S, h) ||
+            (beside && iris_hip_download(m->host_out + slot * n, m->out + slot * n, n * sizeof(float), slot))) {
             fail("layer output");
-            iris_hip_sync();
+            finish_downloads(sent);
             return NULL;
         }
+        if (beside) sent |= 1u << slot;
     }
     /* the caller's memory: its pages are touched while the device works, and
      * each layer's rows are copied in as they arrive. 15.7 MB of fresh pages
