@@ -219,6 +219,7 @@ void *iris_hip_host_malloc(size_t bytes) {
     void *p = nullptr;
     if (!iris_hip_available()) return nullptr;
     if (hipHostMalloc(&p, bytes ? bytes : 256, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();   /* the caller may go on without it */
         iris_set_error("hipHostMalloc(%zu) failed", bytes);
         return nullptr;
     }

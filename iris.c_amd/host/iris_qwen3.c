@@ -51,8 +51,8 @@ struct qwen3_model {
     qlayer_t *L;
     /* work buffers for QWEN3_MAX_SEQ_LEN tokens */
     int *ids;
-    float *x, *out;           /* x [S][h] residual stream; out: the extracted layers [3][S][h] */
-    float *host_out;          /* pinned copy of out, one extracted layer after the other */
+    float *x, *out;           /* x [S][h] residual stream; out: the extracted layers, [3][S][h] or [S][3h] */
+    float *host_out;          /* pinned copy of out, one extracted layer after the other; or NULL */
     uint16_t *a, *qkv, *q, *k, *vt, *attn, *mlp;
     float *rope_cos, *rope_sin;   /* [S][128], value of pair p at 2p and 2p+1 */
     float *rp_cos, *rp_sin;       /* [S][64], value of pair p at p (the attention's Q prologue) */
@@ -237,7 +237,8 @@ static int alloc_work(qwen3_model_t *m) {
     QA(m->ids, S * sizeof(int));
     QA(m->x, S * h * 4);
     QA(m->out, S * 3 * h * 4);
-    if (!(m->host_out = (float *)iris_hip_host_malloc(S * 3 * h * 4))) return -1;
+    /* NULL: the result comes back in one copy at the end */
+    m->host_out = (float *)iris_hip_host_malloc(S * 3 * h * 4);
     QA(m->a, S * h * 2);
     QA(m->qkv, S * (qd + 2 * kd) * 2);
     QA(m->q, S * qd * 2);
@@ -494,8 +495,10 @@ float *qwen3_forward(qwen3_model_t *m, const int *input_ids, const int *attentio
     const int slots = m->mode ? 1 : 3;
     const size_t n = (size_t)S * h;
     /* a small result is not worth the second stream's events (37 tokens, 379
-     * KB: 2810 us with one copy at the end, 2932 with them) */
-    const int beside = slots * n * sizeof(float) >= ((size_t)1 << 20);
+     * KB: 2810 us with one copy at the end, 2932 with them), and without the
+     * pinned memory there is nothing to copy beside: then out holds the
+     * caller's rows */
+    const int beside = m->host_out && slots * n * sizeof(float) >= ((size_t)1 << 20);
     unsigned sent = 0;   /* slots whose download is in flight */
     const iris_norm_args_t first = rms(m, m->L[0].ln1, S);
     if (iris_hip_rownorm(&first)) {
@@ -513,7 +516,7 @@ float *qwen3_forward(qwen3_model_t *m, const int *input_ids, const int *attentio
         /* an extracted layer is copied aside and downloaded while the layers
          * after it run */
         if (slot < 0) continue;
-        if (iris_hip_copy_rows(m->out + slot * n, h, m->x, h, S, h) ||
+        if (iris_hip_copy_rows(m->out + (beside ? slot * n : (size_t)slot * h), beside ? h : text_dim, m->x, h, S, h) ||
             (beside && iris_hip_download(m->host_out + slot * n, m->out + slot * n, n * sizeof(float), slot))) {
             fail("layer output");
             finish_downloads(sent);
@@ -527,10 +530,10 @@ float *qwen3_forward(qwen3_model_t *m, const int *input_ids, const int *attentio
      * 5743 us). */
     float *out = (float *)malloc((size_t)S * text_dim * sizeof(float));
     for (size_t i = 0; out && i < (size_t)S * text_dim; i += 1024) ((volatile float *)out)[i] = 0.0f;
-    int rc = !out || (!beside && iris_hip_memcpy_d2h(m->host_out, m->out, slots * n * sizeof(float)));
-    for (int slot = 0; slot < slots; slot++) {
-        const float *src = m->host_out + (size_t)slot * S * h;
-        if (beside && iris_hip_download_wait(slot)) rc = -1;
+    int rc = !out || (!beside && iris_hip_memcpy_d2h(out, m->out, slots * n * sizeof(float)));
+    for (int slot = 0; beside && slot < slots; slot++) {
+        const float *src = m->host_out + slot * n;
+        if (iris_hip_download_wait(slot)) rc = -1;
         if (rc) continue;
 #pragma omp parallel for schedule(static) num_threads(4) if (S > 64)
         for (int r = 0; r < S; r++) memcpy(out + (size_t)r * text_dim + (size_t)slot * h, src + (size_t)r * h, h * sizeof(float));

@@ -16,15 +16,15 @@ STUBS = r"""
 #include "iris_synth.h"
 #include <stdlib.h>
 #include <string.h>
-int fail_gemm_at = -1, gemms, fail_rows_at = -1, rows_calls, clobbered;
+int fail_gemm_at = -1, gemms, fail_rows_at = -1, rows_calls, clobbered, no_pinned;
 struct { void *dst; const void *src; size_t n; int on; } down[8];
-void reset(void) { memset(down, 0, sizeof(down)); clobbered = 0; fail_gemm_at = fail_rows_at = -1; }
+void reset(void) { memset(down, 0, sizeof(down)); clobbered = no_pinned = 0; fail_gemm_at = fail_rows_at = -1; }
 int pending(void) { int n = 0; for (int i = 0; i < 8; i++) n += down[i].on; return n; }
 int iris_hip_init(int d) { (void)d; return 0; }
 const char *iris_hip_last_error(void) { return "stub"; }
 void *iris_hip_malloc(size_t n) { return calloc(1, n); }
 void iris_hip_free(void *p) { free(p); }
-void *iris_hip_host_malloc(size_t n) { return calloc(1, n); }
+void *iris_hip_host_malloc(size_t n) { return no_pinned ? NULL : calloc(1, n); }
 void iris_hip_host_free(void *p) { free(p); }
 int iris_hip_sync(void) { return 0; }
 int iris_hip_memcpy_h2d(void *d, const void *s, size_t n) { memcpy(d, s, n); return 0; }
@@ -118,9 +118,12 @@ def expect(S, layers):
 
 @pytest.mark.parametrize("mode,layers", [(0, (8, 17, 26)), (1, (LAYERS - 2,))])
 @pytest.mark.parametrize("S", [37, 512])
-def test_rows(lib, S, mode, layers):
-    """Both sides of the 1 MiB line, both modes: the extracted layers side by side."""
+@pytest.mark.parametrize("no_pinned", [0, 1])
+def test_rows(lib, S, mode, layers, no_pinned):
+    """Both sides of the 1 MiB line, both modes: the extracted layers side by
+    side, also where no pinned memory is to be had."""
     lib.reset()
+    set_int(lib, no_pinned=no_pinned)
     m = lib.qwen3_model_create_synthetic(H, 64, 2, 1, LAYERS, 1024, 1)
     assert m
     lib.qwen3_model_set_extraction_mode(m, mode)
