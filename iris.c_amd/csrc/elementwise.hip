@@ -269,26 +269,38 @@ __device__ __forceinline__ void qk_norm_rope_rows(const iris_qkprep_args_t &a, i
         const int nh = which && a.kv_heads ? a.kv_heads : a.heads;
         const uint16_t *src = a.qkv + (size_t)row * a.ld_qkv + (which ? a.col_k : 0) + d0;
         uint16_t *dst = (which ? a.k_out : a.q_out) + (size_t)row * nh * 128 + d0;
-        for (int hb = 0; hb < nh; hb += 4) {
-            const int head = hb + hq;
-            const bool on = head < nh;                        /* uniform per 16-lane group */
-            u16x8 raw = {0, 0, 0, 0, 0, 0, 0, 0};
-            if (on) raw = __builtin_nontemporal_load((const u16x8 *)(src + head * 128));
-            float x[8];
-            float ss = 0.0f;
+        /* two heads per 16-lane group, their loads in flight together; the 16
+         * lanes hold a head's sum alike, so odd lanes take the second's root
+         * and quotient (25 instructions) while even ones take the first's.
+         * Text encode of 37 tokens 2836 -> 2819 us, of 300 5049 -> 5044 */
+        for (int hb = hq; hb < nh; hb += 8) {
+            const bool two = hb + 4 < nh;                     /* uniform per 16-lane group */
+            u16x8 raw[2] = {{0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0, 0}};
+            raw[0] = __builtin_nontemporal_load((const u16x8 *)(src + hb * 128));
+            if (two) raw[1] = __builtin_nontemporal_load((const u16x8 *)(src + (hb + 4) * 128));
+            float x[2][8], ss[2];
 #pragma unroll
-            for (int j = 0; j < 8; j++) { x[j] = bf2f(raw[j]); ss += x[j] * x[j]; }
-            ss = row16_sum(ss);
-            const float inv = 1.0f / sqrtf(ss / 128.0f + a.eps);
-            u16x8 out;
+            for (int i = 0; i < 2; i++) {
+                ss[i] = 0.0f;
 #pragma unroll
-            for (int j = 0; j < 8; j += 2) {
-                const float x0 = x[j] * inv * w[j], x1 = x[j + 1] * inv * w[j + 1];
-                /* fused as written, as in the attention's Q prologue */
-                out[j] = f2bf_hw(__builtin_fmaf(x0, c[j], -(x1 * sn[j])));
-                out[j + 1] = f2bf_hw(__builtin_fmaf(x0, sn[j], x1 * c[j]));
+                for (int j = 0; j < 8; j++) { x[i][j] = bf2f(raw[i][j]); ss[i] += x[i][j] * x[i][j]; }
+                ss[i] = row16_sum(ss[i]);
             }
-            if (on) *(u16x8 *)(dst + head * 128) = out;
+            const int inv2 = __float_as_int(1.0f / sqrtf(((hl & 1) ? ss[1] : ss[0]) / 128.0f + a.eps));
+            const float inv[2] = {__int_as_float(__builtin_amdgcn_mov_dpp(inv2, 0x150, 0xF, 0xF, false)),  /* row_newbcast */
+                                  __int_as_float(__builtin_amdgcn_mov_dpp(inv2, 0x151, 0xF, 0xF, false))};
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                u16x8 out;
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) {
+                    const float x0 = x[i][j] * inv[i] * w[j], x1 = x[i][j + 1] * inv[i] * w[j + 1];
+                    /* fused as written, as in the attention's Q prologue */
+                    out[j] = f2bf_hw(__builtin_fmaf(x0, c[j], -(x1 * sn[j])));
+                    out[j + 1] = f2bf_hw(__builtin_fmaf(x0, sn[j], x1 * c[j]));
+                }
+                if (i == 0 || two) *(u16x8 *)(dst + (hb + 4 * i) * 128) = out;
+            }
         }
     }
 }

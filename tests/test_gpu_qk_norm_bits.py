@@ -38,9 +38,10 @@ def tables(rng, S, rope):
     return (np.cos(ang), np.sin(ang)) if rope else (np.ones((S, 64)), np.zeros((S, 64)))
 
 
-@pytest.mark.parametrize("S,H,split,rope", [(1024, 8, 1024, False), (257, 3, 100, False), (1024, 8, 300, True)])
+@pytest.mark.parametrize("S,H,split,rope", [(1024, 8, 1024, False), (257, 3, 100, False), (1024, 8, 300, True),
+                                            (130, 5, 60, True), (70, 30, 0, True), (3, 1, 2, False)])
 def test_prepared_rows(lib, S, H, split, rope):
-    """2 x 1 M values: a last-bit error of 1 / sqrt in a fifth of the rows moves several over a bf16 rounding line"""
+    """Whole and part-empty rounds of 8 heads. 2 x 1 M values: a last-bit error of 1 / sqrt in a fifth of the rows moves several over a bf16 rounding line"""
     rng = np.random.default_rng(S)
     h, S_pad = H * 128, (S + 63) // 64 * 64
     qkv = rng.integers(-9, 10, (S, 3, H, 128))
