@@ -215,8 +215,9 @@ typedef struct {
 int iris_hip_conv3x3(const iris_conv3x3_t *c);
 /* The same convolution, up to the order of its f32 sums, on 16 x 16 pixel
  * tiles that stage their input once for all nine taps, where that is faster
- * (up 0 and 1, cout a multiple of 128, sides that the tiles do not overshoot
- * by much; splits at most 1), else iris_hip_conv3x3. With a workspace few
+ * (up 0 and 1, cout a multiple of 128, GroupNorm groups of at most 128
+ * channels, fewer or shorter rounds of blocks; splits at most 1), else
+ * iris_hip_conv3x3. With a workspace few
  * tiles are split over the input channels. gn_part gets one row per tile, row
  * by row of tiles; *gn_blocks (if not NULL) receives the number of rows for
  * iris_hip_gn_finalize, at most ceil(H / 16) * ceil(W / 16) or

@@ -1778,6 +1778,16 @@ int conv_params(const iris_conv3x3_t *c, int bnt, GemmParams &P) {
     return 0;
 }
 
+/* Output channels per tile of iris_hip_conv3x3, for arguments conv_params
+ * takes: 128 also where 256 leave half the CUs without a tile (a GroupNorm's
+ * group must stay within one): 128 x 128 pixels out, stride 2, 256 -> 256 (64
+ * tiles of 256) 62 -> 42 us; 64 x 64, 512 -> 512 split by 4 (128) 39 -> 30. */
+int conv_width(const iris_conv3x3_t *c) {
+    const long long tiles = ((long long)c->H * c->W + BM - 1) / BM * (c->cout <= 128 ? 1 : (c->cout + BN - 1) / BN);
+    const bool few = 2 * tiles * (c->splits > 1 ? c->splits : 1) <= iris_cu_count();
+    return c->cout <= 128 || (few && (!c->gn_part || 128 % (c->cout / c->gn_groups) == 0)) ? 128 : BN;
+}
+
 }  // namespace
 
 extern "C" int iris_hip_conv3x3(const iris_conv3x3_t *c) {
@@ -1785,13 +1795,8 @@ extern "C" int iris_hip_conv3x3(const iris_conv3x3_t *c) {
     if (conv_params(c, 0, P)) return -1;
     const iris_gemm_problem_t &p = P.p[0];
     if (p.N <= 0) return 0;
-    /* 128 channels per tile also where 256 leave half the CUs without one (a
-     * GroupNorm's group must stay within a tile): 128 x 128 pixels out, stride
-     * 2, 256 -> 256 (64 tiles of 256) 62 -> 42 us; 64 x 64, 512 -> 512 split by
-     * 4 (128) 39 -> 30. */
-    const bool few = 2LL * P.tiles_m[0] * P.tiles_n[0] * (c->splits > 1 ? c->splits : 1) <= iris_cu_count();
-    const int bnt = p.N <= 128 || (few && (!c->gn_part || 128 % (p.N / c->gn_groups) == 0)) ? 128 : BN;
-    if (few && conv_params(c, bnt, P)) return -1;
+    const int bnt = conv_width(c);
+    if (conv_params(c, bnt, P)) return -1;
     int chunks = 1;
     long long stride = 0;
     P.chunks[0] = 1;
@@ -2140,18 +2145,46 @@ static int conv_tiled(const iris_conv3x3_t *c, int *gn_blocks, uint16_t *bf16_ou
     const int cus = iris_cu_count();
     const long long ty = (c->H + 15) / 16, tx = (c->W + 15) / 16, tiles = ty * tx * (c->cout / 128);
     const double area = (double)c->H * c->W;
-    /* Tiles past one round may overshoot the image by a third (the products
-     * of the overshoot cost time there; at 1.13, 90 x 166, they still win);
-     * within a round they only use idle CUs. */
     /* a GroupNorm group wider than a tile, or no whole number of channels, is the other kernel's to take or refuse */
     const int G = c->gn_part ? c->gn_groups : 0;
     const bool wide = c->gn_part && (G <= 0 || c->cout % G || 128 % (c->cout / G));
-    if (c->cout % 128 || wide || c->ldo % 4 || (((uintptr_t)c->out | (uintptr_t)c->bias) & 15) || tiles >= (1LL << 28) ||
-        (tiles > cus && 256.0 * ty * tx > 1.35 * area))
+    if (c->cout % 128 || wide || c->ldo % 4 || (((uintptr_t)c->out | (uintptr_t)c->bias) & 15) || tiles >= (1LL << 28))
         return other();
     GemmParams chk;
     if (conv_params(c, 128, chk)) return -1;
     const int chunks = c->cin / BK;
+    /* Past one round the kernel with the shorter rounds: tiles of 16 x 16
+     * pixels come in other numbers than row tiles of 256, overshoot the image,
+     * and have half the channels. The estimate (us) is a full round's time by
+     * the 64-channel chunks and the last round's by its fill, fitted to 88
+     * convolutions of 128 to 512 channels and sides of 17 to 1024 pixels, most
+     * within 8 %; 7 more for the other kernel, whose output the pass after it
+     * finds less of in L2 (144 x 144 x 512: apply pass 13 -> 17 us), so that
+     * near ties stay here. Measured, this kernel / the other, bf16 out, 512 ->
+     * 512: 144 x 144 94 / 93, 176 x 176 105 / 112, 180 x 180 (576 tiles / 254)
+     * 145 / 114, 192 x 192 148 / 187, upsampled 180 x 180 138 / 115, 90 x 166
+     * (264 tiles / 236 of 128 channels) 93 / 67, 17 x 640 94 / 62; 360 x 360,
+     * 512 -> 256 248 / 225. With the choice instead of this kernel throughout:
+     * 720 x 720 decode 6367 -> 6157 us, encode 3607 -> 3522, 1328 x 720 decode
+     * 11229 -> 11059.
+     * Within a round a tile's overshoot only uses idle CUs, and a lone chunk
+     * (the layer in front of the decoder, f32 out) is bound by its stores in
+     * both: 144 x 144 x 64 -> 512 28.1 / 28.7, 224 x 224 52.6 / 54.4, 180 x
+     * 180 39.7 / 32.4. */
+    if (tiles > cus && chunks > 1) {
+        const int width = conv_width(c);
+        const long long rows = ((long long)c->H * c->W + BM - 1) / BM * ((c->cout + width - 1) / width);
+        const double epi = c->epi == IRIS_EPI_ADD ? 11.0 : c->epi == IRIS_EPI_F32 ? 5.0 : 0.0;
+        const auto rounds = [&](long long n, double last, int power) {
+            const double r = (double)((n + cus - 1) / cus), fill = (n - (r - 1) * cus) / cus;
+            return r + last * (power == 3 ? fill * fill * fill : fill);
+        };
+        const double tiled = (10.0 + 5.0 * chunks) * (c->up ? 0.94 : 1.0) * (rounds(tiles, 0.2, 1) - 0.12);
+        const double gemm = (width == 128 ? 10.0 + 7.0 * chunks + epi / 2 : 16.0 + 12.0 * chunks + epi) *
+                            (rounds(rows, 0.26, 3) - 0.22) +
+                            7.0 + (bf16_out ? 6.0 * area * c->cout / 4.5e6 + 3.5 : 0.0);   /* the conversion pass */
+        if (gemm < tiled) return other();
+    }
     const bool can = c->ws && !((uintptr_t)c->ws & 15);
     /* Few tiles: half their channels each where twice as many still have a CU
      * (a GroupNorm's group must stay within a tile), and a split over the

@@ -177,6 +177,40 @@ def test_conv3x3_tiled_groups_of_the_other_kernel(lib, cout, G, ok):
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("H,W,cin,cout,up,tiled", [
+    (128, 128, 512, 512, 0, True),     # one round of tiles
+    (144, 144, 512, 512, 0, True),     # 1.27 rounds of tiles, 162 row tiles: 94 us, 93 there and 4 in the pass after
+    (132, 132, 512, 512, 1, True),     # upsampled 90, 92 there
+    (176, 176, 512, 512, 0, True),     # 1.89 rounds: 105, 112 there
+    (180, 180, 512, 512, 0, False),    # 2.25 rounds, 254 row tiles: 145, 114 there
+    (180, 180, 512, 512, 1, False),    # 138, 115 there
+    (192, 192, 512, 512, 0, True),     # 2.25 rounds, 288 row tiles: 148, 187 there
+    (360, 360, 512, 256, 0, False),    # 248, 225 there
+    (360, 360, 256, 128, 0, False),    # 87, 82 there
+    (90, 166, 512, 512, 0, False),     # tiles overshoot: 93, 67 there
+    (17, 640, 512, 512, 0, False),     # by 1.9: 94, 62 there
+])
+def test_conv3x3_tiled_rounds(lib, H, W, cin, cout, up, tiled):
+    """Past one tile per CU the kernel measured faster runs, and gives what the
+    other gives up to the order of the sums and a rounding to bf16."""
+    rng = np.random.default_rng(H)
+    x = rng.standard_normal(((H >> up) * (W >> up) * cin), np.float32)
+    w = rng.standard_normal(cout * 9 * cin, np.float32) / np.float32(np.sqrt(9 * cin))
+    dx, dw = tl.Dev.of(tl.to_bf16(x)), tl.Dev.of(tl.to_bf16(w))
+    outs = []
+    for other in (0, 1):
+        o = tl.Dev(H * W * cout * 2)
+        c = tl.Conv3x3(dx.ptr, dw.ptr, o.ptr, None, H, W, cin, cout, up, cout, EPI_BF16, 1, None, 0, None, 0)
+        assert lib.iris_hip_profile_enable(1) == 0
+        rc = lib.iris_hip_conv3x3(ctypes.byref(c)) if other else lib.iris_hip_conv3x3_tiled(ctypes.byref(c), None)
+        assert rc == 0, lib.iris_hip_last_error()
+        recs = (tl.KernelTime * 4)()
+        assert lib.iris_hip_profile_read(recs, 4) == 1 and lib.iris_hip_profile_enable(0) == 0
+        assert (b"patch" in recs[0].kernel) == (tiled and not other), recs[0].kernel
+        outs.append(tl.bf16_to_f32(o.get(np.uint16, (H, W, cout))))
+    assert tl.rel_l2(outs[0], outs[1]) < 4e-3
+
+
 @pytest.mark.parametrize("H,W,cin,cout,up,split", [
     (173, 190, 128, 128, 0, False),   # 128-channel tiles, ragged
     (61, 50, 128, 256, 0, False),     # 64-channel tiles
