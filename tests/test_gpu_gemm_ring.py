@@ -87,16 +87,51 @@ def test_gemm_ring_bitwise(lib, rows, M, N, K, splits, epi):
     ws.close()
 
 
-@pytest.mark.parametrize("M,N,K,epi", [(1, 6144, 2560, EPI_BF16), (37, 2560, 9728, EPI_GATED_ADD),
-                                       (64, 19456, 2560, EPI_SWIGLU), (65, 3840, 3840, EPI_F32),
-                                       (128, 2560, 4096, EPI_GATED_ADD), (129, 2560, 4096, EPI_GATED_ADD),
-                                       (512, 6144, 2560, EPI_BF16), (256, 128, 3072, EPI_F32_T)])
-def test_gemm_fill_few_rows(lib, M, N, K, epi):
+@pytest.mark.parametrize("rows", [64, 128])
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("shapes", [
+    [(37, 192, 448, EPI_BF16), (128, 320, 448, EPI_F32)],
+    [(1, 128, 64, EPI_F32), (130, 192, 1024, EPI_GATED_ADD), (64, 448, 320, EPI_ADD)],
+    [(65, 64, 640, EPI_SWIGLU), (3, 321, 192, EPI_F32_T), (129, 130, 448, EPI_BF16), (64, 128, 2560, EPI_GATED_ADD)]])
+def test_gemm_ring_several_problems(lib, shapes, splits, rows):
+    """2 to 4 problems of different rows, columns, K and epilogues in one
+    launch, whole and split over K (K of one step is not): each the bits of the
+    two-stage kernel on that problem alone."""
+    ps = [Product(*s) for s in shapes]
+    ws, outs = tl.Dev(WS), []
+    arr = (tl.GemmProblem * len(ps))()
+    for i, p in enumerate(ps):
+        M, N, K = p.dims
+        outs.append(tl.Dev.of(tl.to_bf16(p.x0) if p.bf16 else p.x0))
+        arr[i] = tl.GemmProblem(p.dev[0].ptr, p.dev[1].ptr, outs[i].ptr, None if p.epi == EPI_SWIGLU else p.dev[2].ptr,
+                                M, N, K, K, K, p.ldo, p.epi)
+    assert lib.iris_hip_gemm_ring(arr, len(ps), rows, splits, ws.ptr, WS) == 0, lib.iris_hip_last_error()
+    assert lib.iris_hip_sync() == 0
+    for p, o in zip(ps, outs):
+        want = p.run(lib, lambda pr: lib.iris_hip_gemm_splitk(pr, splits, ws.ptr, WS))
+        assert np.array_equal(o.get(np.uint16 if p.bf16 else np.float32, p.shape), want), p.dims
+    ws.close()
+
+
+@pytest.mark.parametrize("M,N,K,epi,ring", [(1, 6144, 2560, EPI_BF16, True), (37, 2560, 9728, EPI_GATED_ADD, True),
+                                            (64, 19456, 2560, EPI_SWIGLU, True), (65, 3840, 3840, EPI_F32, True),
+                                            (128, 2560, 4096, EPI_GATED_ADD, True),
+                                            (129, 2560, 4096, EPI_GATED_ADD, False),
+                                            (512, 6144, 2560, EPI_BF16, True), (256, 128, 3072, EPI_F32_T, False)])
+def test_gemm_fill_few_rows(lib, M, N, K, epi, ring):
     """The text encoder's and the captions' products around the 128-row line
-    of the rule, through iris_hip_gemm_fill: repeatable, against float64."""
+    of the rule, through iris_hip_gemm_fill: which kernel runs, repeatable,
+    against float64."""
     ws = tl.Dev(WS)
     p = Product(M, N, K, epi)
-    got = [p.run(lib, lambda pr: lib.iris_hip_gemm_fill(pr, ws.ptr, WS)) for _ in range(2)]
+    got = []
+    for _ in range(2):
+        assert lib.iris_hip_profile_enable(1) == 0
+        got.append(p.run(lib, lambda pr: lib.iris_hip_gemm_fill(pr, ws.ptr, WS)))
+        recs = (tl.KernelTime * 4)()
+        n = lib.iris_hip_profile_read(recs, 4)
+        assert lib.iris_hip_profile_enable(0) == 0
+        assert any(b"ring" in r.kernel for r in recs[:n]) == ring, [r.kernel for r in recs[:n]]
     assert np.array_equal(got[0], got[1])
     y = p.exact()
     assert tl.rel_l2(tl.bf16_to_f32(got[0]) if p.bf16 else got[0], y) < (4e-3 if p.bf16 else 1e-5)
