@@ -604,20 +604,26 @@ def run_vae(lib, c, args):
 
     ms_step, wall = timed_steps(lib, step, args)
     lib.iris_vae_gpu_free(v)
-    # the dominant launch shape: 3x3 conv 256 -> 256 at 512x512 (5 per decode)
+    # the 3x3 convolution 256 -> 256 at a quarter of the pixels, with its
+    # GroupNorm sums: bf16 out (2 per decode) and added to the f32 stream (2;
+    # a third leaves its sum in bf16 only)
     H = W = 8 * lh
     cin = cout = 256
     x = tl.Dev(H * W * cin * 2)
     x.put(tl.to_bf16(synth_f32((H * W * cin,), 3)))
     wt = tl.Dev(cout * 9 * cin * 2)
     wt.put(tl.to_bf16(synth_f32((cout * 9 * cin,), 9, 0, 1.0 / 48)))
-    o = tl.Dev(H * W * cout * 4)
-    conv = tl.Conv3x3(x.ptr, wt.ptr, o.ptr, None, H, W, cin, cout, 0, cout, 0, 1, None, 0)
-    c_ms = time_launches(lib, lambda: lib.iris_hip_conv3x3(ctypes.byref(conv)))
-    for d in (x, wt, o, lat, rgb):
+    o, part = tl.Dev(H * W * cout * 4), tl.Dev(H * W // 256 * 32 * 16)
+    assert lib.iris_hip_memset(o.ptr, 0, H * W * cout * 4) == 0
+    lib.iris_hip_conv3x3_tiled.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    kernels = []
+    for epi, key, what in ((1, "conv_256_512", "bf16 out"), (5, "conv_256_512_add", "residual sum")):
+        conv = tl.Conv3x3(x.ptr, wt.ptr, o.ptr, None, H, W, cin, cout, 0, cout, epi, 0, None, 0, part.ptr, 32)
+        c_ms = time_launches(lib, lambda: lib.iris_hip_conv3x3_tiled(ctypes.byref(conv), None))
+        kernels.append(kernel_entry(f"conv3x3_patch_kernel (3x3 conv on pixel tiles): 256->256, 512x512 pixels, {what}",
+                                    c_ms, 2.0 * H * W * cin * cout * 9, 2, key))
+    for d in (x, wt, o, part, lat, rgb):
         d.close()
-    kernels = [kernel_entry("gemm_bf16_kernel<1> (implicit-GEMM 3x3 conv): 256->256, 512x512 pixels", c_ms,
-                            2.0 * H * W * cin * cout * 9, 5, "conv_256_512")]
     cfg = {"workload": c["workload"], "latent": [4 * c["z"], lh, lw], "image": [16 * lh, 16 * lw],
            "z_channels": c["z"], "bottleneck_tokens": 4 * lh * lw}
     return ms_step, wall, vae_flops(c), kernels, cfg, t_load, None, None

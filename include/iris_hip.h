@@ -136,7 +136,8 @@ int iris_hip_gemm_splitk(const iris_gemm_problem_t *problem, int splits, float *
  * workspace holds (splits * M * N floats); otherwise the plain launch. For
  * the products on few rows (a 512-token caption or text stream, a 128-column
  * final projection) that leave most of the chip idle. Products of at most 128
- * rows take iris_hip_gemm_ring's kernel. */
+ * rows with K of 2048 and more take iris_hip_gemm_ring's kernel where its
+ * estimate is lower. */
 int iris_hip_gemm_fill(const iris_gemm_problem_t *problem, float *d_workspace, size_t workspace_bytes);
 
 /* No counterpart in the reference. iris_hip_gemm_fill over up to 4
@@ -153,9 +154,10 @@ int iris_hip_gemm_fill_n(const iris_gemm_problem_t *problems, int n_problems, fl
 
 /* No counterpart in the reference. The launch on tiles of 64 or 128 rows by
  * 128 columns whose loads run in waves of their own, several K steps ahead:
- * what iris_hip_gemm_fill and _fill_n take for products of at most 128 rows
- * (a short prompt, a caption) and, unsplit, for one whose 128 x 128 tiles
- * fill most of one round. splits and the workspace as iris_hip_gemm_splitk
+ * what iris_hip_gemm_fill and _fill_n take, given a workspace, K of 2048 and
+ * more, no second K segment and an estimate below the two-stage kernel's, for
+ * products of at most 128 rows (a short prompt, a caption) and, unsplit, for
+ * one whose 128 x 128 tiles fill most of one round. splits and the workspace as iris_hip_gemm_splitk
  * (every problem split alike); results equal it and iris_hip_gemm bit for
  * bit. No second K segment. */
 int iris_hip_gemm_ring(const iris_gemm_problem_t *problems, int n_problems, int rows, int splits, float *d_workspace,

@@ -775,7 +775,7 @@ __global__ __launch_bounds__(NT) void gemm_bf16_kernel(const GemmParams P) {
  * the address unit (16 clocks per 1 KiB load), so where the computing waves
  * also load, a step takes the sum of its load issue, products and fragment
  * reads; with waves of their own the loads cost the products nothing, and
- * NS - 1 steps are in flight (72 to 120 KiB per CU) against the latency of
+ * NS - 1 steps are in flight (96 or 120 KiB per CU) against the latency of
  * weights that come from HBM.
  *
  * One barrier per K step. A computing wave runs step t's first 32-wide half
@@ -1507,19 +1507,28 @@ namespace {
 
 /* The faster plan of gemm_ring_kernel for these problems: at most 128 rows
  * each, in up to one round of blocks, or one problem whose 128 x 128 tiles
- * fill most of a round unsplit; K of 2048 and more (32 steps: a shorter K
- * costs a launch either way, and keeps the chunks of the two-stage plan
- * whatever the number of rows). Elsewhere its tiles load more bytes per
- * product than the larger ones and lose (measured, cold weights, us against
- * the two-stage kernel's plans: 512 x 2560 x 9728 45.7 / 45.4, 768 x 18432 x
- * 3072 122 / 69). The estimate (us): K steps per block times a step of the
- * tile, plus launch, prologue and epilogue, plus the reduce pass; not less
- * than the weights' read at the device's copy rate. Measured against it, us,
- * cold weights (two-stage plan -> this kernel): 37 rows, N x K 6144 x 2560
- * 20.4 -> 15.8, 2560 x 4096 19.5 -> 14.8, 19456 x 2560 SwiGLU 32.5 -> 26.1,
- * 2560 x 9728 26.7 -> 20.8; 96 rows, 3840 x 3840 23.3 -> 18.0; 128 rows,
- * 2560 x 9728 30.1 -> 24.4; 512 x 6144 x 2560 (192 tiles, no reduce pass)
- * 39.4 -> 31.6. */
+ * fill most of a round unsplit; K of 2048 and more (32 steps). Elsewhere its
+ * tiles load more bytes per product than the larger ones and lose (measured,
+ * cold weights, us, two-stage kernel's plan / this kernel unsplit: 512 x 2560
+ * x 4096 32.7 / 40.8, 384 x 2560 x 9728 42.3 / 98.3; 768 x 18432 x 3072 69 /
+ * 122). The estimate (us): K steps per block times a step of the tile, plus
+ * launch, prologue and epilogue, plus the reduce pass; not less than the
+ * weights' read at the device's copy rate. It and the two-stage kernel's are
+ * each fitted as a whole to their own kernel's times (a reduce pass is 3.5 in
+ * this one and 6 in that one) and know nothing of the row pass that may take
+ * the reduce's place. Measured, cold weights, us between events (two-stage
+ * plan -> this kernel): 37 rows, N x K 6144 x 2560 22.8 -> 19.0, 2560 x 4096
+ * 23.2 -> 19.3, 19456 x 2560 SwiGLU 36.6 -> 28.1, 2560 x 9728 30.3 -> 24.0;
+ * 96 rows, 3840 x 3840 26.0 -> 20.6; 128 rows, 2560 x 9728 34.4 -> 30.3; 512
+ * x 6144 x 2560 (192 tiles, no reduce pass) 42.2 -> 33.1, 385 rows 41.3 ->
+ * 25.7. Nowhere in 84 shapes of 8 to 128 rows is the choice slower than the
+ * two-stage plan by more than the runs differ. It leaves gains: K below 2048
+ * keeps the two-stage plan, whose chunk count does not depend on the number of
+ * rows, though this kernel is faster there too (128 x 3840 x 1024 21.8 / 11.2,
+ * 37 x 3840 x 1536 19.3 / 17.3); 65 x 19456 x 2560 38.1 / 31.9 and 37 x 20480
+ * x 3840 46.2 / 37.3 fall to the estimate's 3 % margin and floor; one problem
+ * of 257 to 384 rows by N 6144 (144 tiles) is below the line of 60 % of a
+ * round, 34.9 / 27.7 at 300. */
 struct RingPlan {
     int ring, splits;
     double us;
@@ -1840,14 +1849,14 @@ namespace {
  * step's products. Here the tile's pixels and their halo (18 x 18, or 10 x 10
  * before the upsample) are staged once per 64 channels and all nine taps read
  * their fragments from that patch; only the weights (16 KiB per step) stream:
- * 189 KiB per 64 channels instead of 432. The tile then leaves through LDS,
- * the residual of IRIS_EPI_ADD in flight while it is staged. Measured against
- * the implicit GEMM, us: 1024 x 1024, 128 -> 128 with the residual 498 -> 367
- * (f32 stream in and out: 210 of it), bf16 out 342 -> 311, 256 -> 128 619 ->
- * 497; 512 x 512, 512 -> 256 467 -> 429 (1.44 PFLOP/s); 256 x 256 x 512
- * upsampled 219 -> 196 (1.58); 128 x 128, 512 -> 512 80.5 -> 53.8. The direct
- * stores of the accumulators took 614 where it takes 367: 64-byte pieces,
- * behind a load each.
+ * 185 KiB per 64 channels (192 with the loads past the patch's end) instead of
+ * 432. The tile then leaves through LDS, the residual of IRIS_EPI_ADD in
+ * flight while it is staged. Measured against the implicit GEMM, us: 1024 x
+ * 1024, 128 -> 128 with the residual 498 -> 367 (f32 stream in and out: 210 of
+ * it), bf16 out 342 -> 311, 256 -> 128 619 -> 497; 512 x 512, 512 -> 256 467
+ * -> 429 (1.44 PFLOP/s); 256 x 256 x 512 upsampled 219 -> 196 (1.58); 128 x
+ * 128, 512 -> 512 80.5 -> 53.8. The direct stores of the accumulators took 614
+ * where it takes 367: 64-byte pieces, behind a load each.
  *
  * 8 waves as in gemm_ring_kernel: waves 0..3 compute (2x2, wave tile 8 pixel
  * rows x TN / 2 channels), waves 4..7 load, one barrier per K step (a tap of a
