@@ -138,6 +138,16 @@ struct AttnSeg {
 /* s_waitcnt immediate: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8 */
 constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8); }
 
+/* lane n (0..7, constant) of each row of 16 lanes, in all of them */
+__device__ __forceinline__ float row16_lane(int v, int n) {
+    switch (n) {   /* row_newbcast:n */
+#define ROW_LANE(i) case i: return __int_as_float(__builtin_amdgcn_mov_dpp(v, 0x150 + (i), 0xF, 0xF, false))
+        ROW_LANE(0); ROW_LANE(1); ROW_LANE(2); ROW_LANE(3); ROW_LANE(4); ROW_LANE(5); ROW_LANE(6);
+        default: ROW_LANE(7);
+#undef ROW_LANE
+    }
+}
+
 template <int FEAT, int NWV>
 __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float scale_log2, int nqb, const int L,
                                              const int t0, int tn, const AttnSplit &sp, const AttnSeg sg) {
@@ -291,45 +301,46 @@ __device__ __forceinline__ void attn_segment(const iris_attn_args_t &a, float sc
          * the line between the two (row order: set A first) */
         const bool mixed = wave_q0 < a.qn_split && wave_q0 + QW > a.qn_split;
         float4 ww0 = wave_q0 < a.qn_split ? wa0 : wb0, ww1 = wave_q0 < a.qn_split ? wa1 : wb1;
-        /* the 16 lanes of a row hold its sum alike: each takes one of the
-         * 8 passes' root and quotient (25 instructions) for all of them: 37
-         * causal queries 11.2 -> 10.5 us, 512 21.6 -> 20.9, 768 24.0 -> 23.7 */
-        float s8[8];
+        /* the 16 lanes of a row hold its sum alike: each takes one of PB
+         * passes' root and quotient (25 instructions) for all of them: 37
+         * causal queries 11.2 -> 10.5 us, 512 21.6 -> 20.9, 768 24.0 -> 23.7.
+         * The rows of PB passes are held in f32 meanwhile; the balanced
+         * schedule's kernel has no registers for that and takes each pass by
+         * itself (8 at a time spilled 68 bytes: 1536 x 2 queries, 32 heads
+         * 108 -> 113 us) */
+        constexpr int PB = (FEAT & F_SPLIT) ? 1 : 8;
 #pragma unroll
-        for (int pass = 0; pass < 8; pass++) {
-            float ss = 0.0f;
+        for (int p0 = 0; p0 < 8; p0 += PB) {
+            float x[PB][8], ss[PB];
 #pragma unroll
-            for (int j = 0; j < 8; j++) { const float v = bf2f(raw[pass][j]); ss += v * v; }
-            s8[pass] = row16_sum(ss);
-        }
+            for (int p = 0; p < PB; p++) {
+                ss[p] = 0.0f;
 #pragma unroll
-        for (int w = 4; w; w >>= 1)
-#pragma unroll
-            for (int i = 0; i < w; i++) s8[i] = (hl & w) ? s8[i + w] : s8[i];
-        const int inv8 = __float_as_int(1.0f / sqrtf(s8[0] / 128.0f + a.qn_eps));
-        float invs[8];
-#define ROW_LANE(n) invs[n] = __int_as_float(__builtin_amdgcn_mov_dpp(inv8, 0x150 + (n), 0xF, 0xF, false)) /* row_newbcast */
-        ROW_LANE(0); ROW_LANE(1); ROW_LANE(2); ROW_LANE(3); ROW_LANE(4); ROW_LANE(5); ROW_LANE(6); ROW_LANE(7);
-#undef ROW_LANE
-#pragma unroll
-        for (int pass = 0; pass < 8; pass++) {
-            const int rw = pass * 4 + rl, row = wave_q0 + rw;
-            const float inv = invs[pass];
-            float x[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) x[j] = bf2f(raw[pass][j]);
-            if (mixed && row >= a.qn_split) { ww0 = wb0; ww1 = wb1; }
-            const float ww[8] = {ww0.x, ww0.y, ww0.z, ww0.w, ww1.x, ww1.y, ww1.z, ww1.w};
-            const float c[4] = {c4[pass].x, c4[pass].y, c4[pass].z, c4[pass].w};
-            const float sn[4] = {s4[pass].x, s4[pass].y, s4[pass].z, s4[pass].w};
-            u16x8 out;
-#pragma unroll
-            for (int j = 0; j < 8; j += 2) {
-                const float x0 = x[j] * inv * ww[j], x1 = x[j + 1] * inv * ww[j + 1];
-                out[j] = f2bf_hw(__builtin_fmaf(x0, c[j >> 1], -(x1 * sn[j >> 1])));
-                out[j + 1] = f2bf_hw(__builtin_fmaf(x0, sn[j >> 1], x1 * c[j >> 1]));
+                for (int j = 0; j < 8; j++) { x[p][j] = bf2f(raw[p0 + p][j]); ss[p] += x[p][j] * x[p][j]; }
+                ss[p] = row16_sum(ss[p]);
             }
-            *(u16x8 *)(qs + rw * KSTR + d0) = out;
+#pragma unroll
+            for (int w = PB / 2; w; w >>= 1)
+#pragma unroll
+                for (int i = 0; i < w; i++) ss[i] = (hl & w) ? ss[i + w] : ss[i];
+            const int inv8 = __float_as_int(1.0f / sqrtf(ss[0] / 128.0f + a.qn_eps));
+#pragma unroll
+            for (int p = 0; p < PB; p++) {
+                const int rw = (p0 + p) * 4 + rl, row = wave_q0 + rw;
+                const float inv = row16_lane(inv8, p);
+                if (mixed && row >= a.qn_split) { ww0 = wb0; ww1 = wb1; }
+                const float ww[8] = {ww0.x, ww0.y, ww0.z, ww0.w, ww1.x, ww1.y, ww1.z, ww1.w};
+                const float4 cv = c4[p0 + p], sv = s4[p0 + p];
+                const float c[4] = {cv.x, cv.y, cv.z, cv.w}, sn[4] = {sv.x, sv.y, sv.z, sv.w};
+                u16x8 out;
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) {
+                    const float x0 = x[p][j] * inv * ww[j], x1 = x[p][j + 1] * inv * ww[j + 1];
+                    out[j] = f2bf_hw(__builtin_fmaf(x0, c[j >> 1], -(x1 * sn[j >> 1])));
+                    out[j + 1] = f2bf_hw(__builtin_fmaf(x0, sn[j >> 1], x1 * c[j >> 1]));
+                }
+                *(u16x8 *)(qs + rw * KSTR + d0) = out;
+            }
         }
         __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));   /* the wave's own LDS writes, read by its other lanes */
 #pragma unroll
